@@ -169,6 +169,12 @@ struct BackwardParams {
 // Each launcher returns the launch status; `name` receives the kernel's
 // name for the profiler.
 hipError_t launch_select(const SelectParams& p, int dtype, bool from_scores, hipStream_t s);
+// The score pass by storage type (one translation unit each), and over
+// caller-given scores.
+hipError_t launch_select_bf16(const SelectParams& p, hipStream_t s);
+hipError_t launch_select_f16(const SelectParams& p, hipStream_t s);
+hipError_t launch_select_f32(const SelectParams& p, hipStream_t s);
+hipError_t launch_select_scores(const SelectParams& p, hipStream_t s);
 // LDS bytes of one select block holding `cap` candidate keys per row.
 size_t select_lds_bytes(const Dims& d, int dtype, bool from_scores, int cap);
 // Candidate keys per row that fit `max_lds` bytes (k + 32 at most; -1 if

@@ -20,8 +20,8 @@ BUILD = os.path.join(ROOT, "_build")
 LIBDIR = os.path.join(PKG_DIR, "lib")
 LIB = os.path.join(LIBDIR, "libadasplash.so")
 
-SOURCES = ["select.hip", "exact.hip", "compact.hip", "forward.hip", "backward.hip", "sparse_bwd.hip",
-           "capi.cpp"]
+SOURCES = ["sparse_bwd.hip", "select_bf16.hip", "select_f16.hip", "select_f32.hip", "forward.hip",
+           "backward.hip", "exact.hip", "select.hip", "compact.hip", "capi.cpp"]
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}",

@@ -135,3 +135,31 @@ def test_select_overflow_rounds_bit_exact(dev, k, min_rounds, with_topk):
     assert rounds >= min_rounds, rounds
     sel, c = _oracle(S, idx, idx, k, 1.5)
     _compare(st, sel, c)
+
+
+@pytest.mark.parametrize("with_topk", [True, False], ids=["topk", "values"])
+@pytest.mark.parametrize("k", [1, 8, 64, 100, 128])
+def test_select_ties_beyond_the_list_bit_exact(dev, k, with_topk):
+    """Rows whose candidates tie at the score clamp in numbers around and far
+    beyond the list's capacity (a row is then done without another sweep
+    when every left-out tie comes after the kept ones), and, in the last
+    third of the rows, tied candidates below better ones that arrive late
+    (another sweep must follow).  One oracle, bit for bit."""
+    N = 1100
+    rng = np.random.default_rng(k)
+    S = rng.normal(size=(1, N, N)).astype(np.float32)
+    cap = k + max(32, k * 3 // 4)
+    for i in range(N):
+        m = rng.integers(max(1, cap - 8), cap + 9) if i % 2 else N // 2
+        at = rng.choice(N, size=min(N, m), replace=False)
+        if i < 2 * N // 3:
+            S[0, i, at] = 12.0 + rng.random(at.size)    # clamped to 10
+        else:
+            S[0, i, at] = 5.0
+            S[0, i, -min(N, 2 * k):] = 6.0 + 0.25 * rng.integers(0, 3, size=min(N, 2 * k))
+    qidx = torch.full((1, N), N - 1, dtype=torch.int32)
+    kidx = causal_idx(1, N)
+    print(f"[select] ties beyond the list k={k} topk={with_topk}", flush=True)
+    st = _run(dev, S, qidx, kidx, k, 1.5, 1, 1, with_topk)
+    sel, c = _oracle(S, qidx, kidx, k, 1.5)
+    _compare(st, sel, c)
