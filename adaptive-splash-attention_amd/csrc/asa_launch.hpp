@@ -85,7 +85,8 @@ struct SelectParams {
   float* topk_val;        // optional
   float* tkv;             // workspace: sorted top-k values, [k][BH * NQ]
   int2* kbounds;          // workspace: (min, max) position per key block, [BH * nKB]
-  int cap;                // candidate keys per row in LDS (select_capacity)
+  int waves, cap;         // score pass: as in SelectPlan
+  bool ring;
   int lcap;               // refine pass: listed keys per row in LDS (refine_list_capacity)
   uint32_t* status;       // optional per-call status word (kStatus* bits), zeroed by bounds_kernel
 };
@@ -175,11 +176,16 @@ hipError_t launch_select_bf16(const SelectParams& p, hipStream_t s);
 hipError_t launch_select_f16(const SelectParams& p, hipStream_t s);
 hipError_t launch_select_f32(const SelectParams& p, hipStream_t s);
 hipError_t launch_select_scores(const SelectParams& p, hipStream_t s);
-// LDS bytes of one select block holding `cap` candidate keys per row.
-size_t select_lds_bytes(const Dims& d, int dtype, bool from_scores, int cap);
-// Candidate keys per row that fit `max_lds` bytes (k + 32 at most; -1 if
-// not even k + 8 fit).
-int select_capacity(const Dims& d, int dtype, bool from_scores, size_t max_lds);
+// How the score pass runs: waves per block (4 or 8), whether its sweeps read
+// K through LDS rings, and the candidate keys per row that its lists hold
+// in `max_lds` bytes of LDS (cap -1: not even k + 4 fit; `needs` bytes).
+struct SelectPlan {
+  int waves;
+  bool ring;
+  int cap;
+  size_t needs;
+};
+SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_lds);
 hipError_t launch_bounds(const SelectParams& p, hipStream_t s);
 hipError_t launch_tau(const SelectParams& p, hipStream_t s);
 // Exact-threshold pass (tau mode "exact"): after launch_tau, before

@@ -284,20 +284,19 @@ int device_cus(int* cus) {
   return ASA_OK;
 }
 
-// Candidate capacity per row of the select kernel on the current device
-// (*cap), or an error when even the smallest capacity does not fit its LDS.
-int select_cap(const Shape& s, bool from_scores, int* cap) {
+// The select kernel's plan on the current device, or an error when even
+// the smallest candidate capacity does not fit its LDS.
+int select_plan_of(const Shape& s, bool from_scores, asa::SelectPlan* plan) {
   int dev = 0, max_lds = 0;
   if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (int rc = check_hip(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock,
                                                dev),
                          "hipDeviceGetAttribute"))
     return rc;
-  const asa::Dims d = dims_of(s);
-  *cap = asa::select_capacity(d, s.dtype, from_scores, size_t(max_lds));
-  if (*cap < 0)
+  *plan = asa::select_plan(dims_of(s), s.dtype, from_scores, size_t(max_lds));
+  if (plan->cap < 0)
     return fail(ASA_ERR_UNSUPPORTED, "k_keep %d needs %zu bytes of LDS per block, device has %d",
-                s.k, asa::select_lds_bytes(d, s.dtype, from_scores, s.k + 8), max_lds);
+                s.k, plan->needs, max_lds);
   return ASA_OK;
 }
 
@@ -324,7 +323,11 @@ int run_select(const Shape& sh, const void* q, const void* k, const float* score
   asa::SelectParams sp{};
   sp.tkv = static_cast<float*>(workspace);
   sp.kbounds = reinterpret_cast<int2*>(static_cast<char*>(workspace) + tkv_bytes(sh));
-  if (int rc = select_cap(sh, scores != nullptr, &sp.cap)) return rc;
+  asa::SelectPlan plan;
+  if (int rc = select_plan_of(sh, scores != nullptr, &plan)) return rc;
+  sp.waves = plan.waves;
+  sp.ring = plan.ring;
+  sp.cap = plan.cap;
   sp.d = dims_of(sh);
   if (sh.exact) {
     // the refine pass's key lists: checked before anything is launched

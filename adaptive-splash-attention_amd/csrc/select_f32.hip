@@ -1,4 +1,4 @@
-// Score pass (select_kernel.hpp) for fp32 operands and for caller-given scores, and its LDS sizes.
+// Score pass (select_kernel.hpp) for fp32 operands and for caller-given scores, and its plan.
 #include "select_kernel.hpp"
 
 namespace asa {
@@ -9,21 +9,30 @@ hipError_t launch_select_scores(const SelectParams& p, hipStream_t s) {
   return launch_r<float, 64, kGivenScores>(p, s);
 }
 
-size_t select_lds_bytes(const Dims& d, int dtype, bool from_scores, int cap) {
-  (void)dtype;
-  (void)from_scores;
-  return size_t(sel_layout(d.k, cap, d.nKB).total);
-}
-
-int select_capacity(const Dims& d, int dtype, bool from_scores, size_t max_lds) {
-  // k + 32 keys per row holds the candidates of random rows with room to
-  // spare up to k = 42, and 1.75 k above (the floor's slack grows with k; at
-  // k = 64 two blocks still share a compute unit, above it one runs either
-  // way); less still works (overflow rounds), as long as it exceeds k.
-  int cap = d.k + (d.k * 3 / 4 > 32 ? d.k * 3 / 4 : 32);
-  if (cap > 256) cap = 256;
-  while (cap > d.k && select_lds_bytes(d, dtype, from_scores, cap) > max_lds) cap -= 8;
-  return cap > d.k ? cap : -1;
+SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_lds) {
+  // Rings: 16-bit inputs, hd = D, raw dots (launch_ring).
+  const bool raw = !from_scores && d.scale > 0.0f;
+  const bool ring = raw && dtype != kElemF32 && d.hd == d.D;
+  // Eight waves where the lists leave room for one block per compute unit
+  // only: above k = 64, and above k = 42 at d = 128 beside the rings (two
+  // 4-wave blocks fit below; 1x16x8192, d = 128, k = 32: 432 against 495 us
+  // with eight).  1x8x32768, d = 128, k = 128: 4.9 -> 3.7 ms.  fp32 at
+  // d = 128 holds 128 registers of Q and would spill at two waves per SIMD.
+  const bool wide = raw && (d.k > 64 || (d.k > 42 && ring && d.D == 128)) &&
+                    !(dtype == kElemF32 && d.D == 128);
+  const struct { int waves; bool ring; } tries[] = {{wide ? 8 : 4, ring}, {4, ring}, {4, false}};
+  for (const auto& t : tries) {
+    auto bytes = [&](int cap) { return size_t(sel_layout(d.k, cap, d.nKB, t.waves, t.ring ? d.D : 0).total); };
+    // k + 32 keys per row hold the candidates of random rows with room to
+    // spare up to k = 42, and 1.75 k above (the floor's slack grows with
+    // k); less still works (overflow rounds), as long as it exceeds k.
+    int cap = d.k + (d.k * 3 / 4 > 32 ? d.k * 3 / 4 : 32);
+    while (cap > d.k && bytes(cap) > max_lds) cap -= 4;
+    if (cap <= d.k) cap = d.k + 4;  // the least taken
+    if (bytes(cap) <= max_lds) return SelectPlan{t.waves, t.ring, cap, 0};
+    if (t.waves == 4 && !t.ring) return SelectPlan{4, false, -1, bytes(cap)};
+  }
+  return SelectPlan{4, false, -1, 0};
 }
 
 }  // namespace asa

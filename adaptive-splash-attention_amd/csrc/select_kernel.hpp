@@ -4,22 +4,22 @@
 //
 // Reference: build_mask_kernel + insert_topk + entmax_threshold
 // (adasplashattention.cu:35-217), one thread per query that scans every key
-// and keeps a sorted top-k by insertion.  Here one 256-thread block owns one
-// 64-row query block of one (batch, head).  During the sweeps the waves
-// split the keys, not the rows: wave w loads keys 16w..16w+15 of each
-// visible key tile straight from L2 into MFMA operand registers (KQuarter,
-// two tiles in flight, no barrier per tile; with 16-bit inputs sweep 1
-// reads them through a per-wave LDS ring filled by global_load_lds) and
-// scores them against all 64 rows.  The top-k is found in two sweeps over the
+// and keeps a sorted top-k by insertion.  Here one block of 4 or 8 waves
+// owns one 64-row query block of one (batch, head).  During the sweeps the
+// waves split the keys, not the rows: a wave takes 16 keys of each of its
+// visible key tiles, from per-wave LDS rings filled by global_load_lds
+// (16-bit inputs at hd = D) or straight from L2 into MFMA operand registers
+// (KQuarter, two tiles in flight), without a barrier per tile, and scores
+// them against all 64 rows.  The top-k is found in two sweeps over the
 // visible key blocks instead of by insertion:
 //
-//   sweep 1  every score updates one of 64*R running "class maxima" of its
-//            row (one v_med3 per score; class = key offset in the tile x
-//            tile ordinal mod R).  Distinct classes hold distinct keys, so
-//            if at least k class maxima are >= x, at least k keys score
-//            >= x, and every top-k key scores >= x.  The class maxima meet
-//            in LDS and an 8-step bisection per row (wave w: rows
-//            16w..16w+15) finds such an x close to the k-th largest.
+//   sweep 1  every score updates one of 128 or 256 running "class maxima" of
+//            its row (one v_med3 per score; class = key offset in the wave's
+//            tile x tile ordinal mod R).  Distinct classes hold distinct
+//            keys, so if at least k class maxima are >= x, at least k keys
+//            score >= x, and every top-k key scores >= x.  The class maxima
+//            meet in LDS and a bisection per row finds such an x close to
+//            the k-th largest.
 //   sweep 2  the scores are recomputed and every key scoring >= x is
 //            appended, as (index, score bits), to the row's list in LDS
 //            (about 1.05-1.15 k keys per row on random data).  If a row
@@ -60,21 +60,28 @@ namespace asa {
 namespace {
 
 
-constexpr int kThreads = 256;  // four waves of 16 query rows
-
 __device__ __forceinline__ int wave_min(int v) { return wave_reduce_minmax<false>(v); }
 __device__ __forceinline__ int wave_max(int v) { return wave_reduce_minmax<true>(v); }
-// Reductions over the 4 lanes (L, L^16, L^32, L^48) that share a row.
-__device__ __forceinline__ int group_sum(int v) {
-  return int(group_reduce_bits(uint32_t(v), [](uint32_t x, uint32_t y) { return x + y; }));
+// Reductions over the NW lanes (4 or 8, equal modulo 64 / NW) that share a
+// row of the floor search.
+template <int NW, typename F>
+__device__ __forceinline__ uint32_t row_reduce(uint32_t v, F op) {
+  if constexpr (NW == 8) v = op(v, lane_xor<8>(v));
+  return group_reduce_bits(v, op);
 }
-__device__ __forceinline__ float group_min(float v) {
-  return __uint_as_float(group_reduce_bits(__float_as_uint(v), [](uint32_t x, uint32_t y) {
+template <int NW>
+__device__ __forceinline__ int row_sum(int v) {
+  return int(row_reduce<NW>(uint32_t(v), [](uint32_t x, uint32_t y) { return x + y; }));
+}
+template <int NW>
+__device__ __forceinline__ float row_min(float v) {
+  return __uint_as_float(row_reduce<NW>(__float_as_uint(v), [](uint32_t x, uint32_t y) {
     return __float_as_uint(fminf(__uint_as_float(x), __uint_as_float(y)));
   }));
 }
-__device__ __forceinline__ float group_max(float v) {
-  return __uint_as_float(group_reduce_bits(__float_as_uint(v), [](uint32_t x, uint32_t y) {
+template <int NW>
+__device__ __forceinline__ float row_max(float v) {
+  return __uint_as_float(row_reduce<NW>(__float_as_uint(v), [](uint32_t x, uint32_t y) {
     return __float_as_uint(fmaxf(__uint_as_float(x), __uint_as_float(y)));
   }));
 }
@@ -93,16 +100,10 @@ __device__ __forceinline__ float opaque_inf() {
   asm("" : "+v"(v));
   return v;
 }
-// Smallest / largest of a 64-bit value over the wave, in scalar registers.
+// Smallest / largest of a 32-bit unsigned value over the wave.
 template <bool kMax>
-__device__ __forceinline__ uint64_t wave_minmax64(uint64_t v) {
-  for (int o = 1; o < kWave; o <<= 1) {
-    const uint64_t y = (uint64_t(uint32_t(__shfl_xor(int(v >> 32), o, kWave))) << 32) |
-                       uint32_t(__shfl_xor(int(v), o, kWave));
-    v = (kMax ? y > v : y < v) ? y : v;
-  }
-  return (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(v >> 32)))) << 32) |
-         uint32_t(__builtin_amdgcn_readfirstlane(int(v)));
+__device__ __forceinline__ uint32_t wave_minmax_u32(uint32_t v) {
+  return uint32_t(wave_reduce_minmax<kMax>(int(v ^ 0x80000000u))) ^ 0x80000000u;
 }
 // c + (x >= t).
 __device__ __forceinline__ uint32_t count_ge(uint32_t c, float x, float t) {
@@ -205,6 +206,13 @@ __device__ __forceinline__ float sweep_floor(float th, bool exact, float scale) 
 }
 
 
+// 16 bytes per lane from `src` to LDS at dst + 16 * lane (global_load_lds).
+// Outside the kernel template: with a template-dependent pointer the host
+// pass drops the kernel's launch stub.
+__device__ __forceinline__ void lds_dma16(const unsigned char* src, unsigned char* dst) {
+  __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)(dst), 16, 0, 0);
+}
+
 enum SweepMode : int {
   kRawDots = 0,     // MFMA dot products, scale > 0: filters on raw dots
   kExactScores = 1, // MFMA dot products converted to exact scores (scale <= 0)
@@ -228,28 +236,16 @@ template <typename T, int D> struct KQuarter;
 template <typename T, int D> struct KQuarter16 {
   using V8 = typename Half<T>::v8;
   V8 a[D / 32];
-  // Keys >= NK read key 0 instead: they lie in partially visible tiles,
-  // where the visibility test discards their scores, so no zeroing (and no
-  // wait for the load where it is issued) is needed.  (This register path
-  // loads 16 half rows per instruction, a third of the L2 rate of whole-row
-  // loads; a whole-row load with the operands rebuilt by two DPP row
-  // rotations per register measured the same sweep time, which the
-  // candidate appends, not the loads, set.)
-  // KL (KLayout): rows of exactly D elements (kKDense), or rows snb bytes
-  // apart (32-bit offsets from the head's first row, which the C ABI
-  // bounds below 2^31) with hd = D (kKRows) or with columns >= hd read as
-  // zero (kKGeneral).
+  // `src`: the tile's first row plus the lane's byte offset (its key's row,
+  // 16 g bytes in).  (This register path loads 16 half rows per instruction,
+  // a third of the L2 rate of whole-row loads; a whole-row load with the
+  // operands rebuilt by two DPP row rotations per register measured the same
+  // sweep time, which the candidate appends, not the loads, set.)  KL
+  // (KLayout): with kKGeneral columns >= hd read as zero.
   template <int KL>
-  __device__ __forceinline__ void load(const T* Kb, int key, int NK, uint32_t snb, int hd, int g) {
-    const int kk = key < NK ? key : 0;
-    if constexpr (KL != kKDense) {
-      const unsigned char* src = reinterpret_cast<const unsigned char*>(Kb) + (uint32_t(kk) * snb + 16u * g);
-      for (int s = 0; s < D / 32; ++s)
-        a[s] = KL == kKRows || 32 * s + 8 * g < hd ? *reinterpret_cast<const V8*>(src + 64 * s) : V8{};
-    } else {
-      const T* src = Kb + size_t(kk) * D + 8 * g;
-      for (int s = 0; s < D / 32; ++s) a[s] = *reinterpret_cast<const V8*>(src + 32 * s);
-    }
+  __device__ __forceinline__ void load(const unsigned char* tile, uint32_t off, int hd, int g) {
+    for (int s = 0; s < D / 32; ++s)
+      a[s] = KL != kKGeneral || 32 * s + 8 * g < hd ? *reinterpret_cast<const V8*>(tile + (off + 64u * s)) : V8{};
   }
   __device__ __forceinline__ void product(f32x4 (&acc)[4], const RowFrag<T, D> (&qf)[4]) const {
     for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -262,16 +258,9 @@ template <int D> struct KQuarter<h16, D> : KQuarter16<h16, D> {};
 template <int D> struct KQuarter<float, D> {
   f32x4 a[D / 16];
   template <int KL>
-  __device__ __forceinline__ void load(const float* Kb, int key, int NK, uint32_t snb, int hd, int g) {
-    const int kk = key < NK ? key : 0;
-    if constexpr (KL != kKDense) {
-      const unsigned char* src = reinterpret_cast<const unsigned char*>(Kb) + (uint32_t(kk) * snb + 16u * g);
-      for (int j = 0; j < D / 16; ++j)
-        a[j] = KL == kKRows || 16 * j + 4 * g < hd ? *reinterpret_cast<const f32x4*>(src + 64 * j) : f32x4{};
-    } else {
-      const float* src = Kb + size_t(kk) * D + 4 * g;
-      for (int j = 0; j < D / 16; ++j) a[j] = *reinterpret_cast<const f32x4*>(src + 16 * j);
-    }
+  __device__ __forceinline__ void load(const unsigned char* tile, uint32_t off, int hd, int g) {
+    for (int j = 0; j < D / 16; ++j)
+      a[j] = KL != kKGeneral || 16 * j + 4 * g < hd ? *reinterpret_cast<const f32x4*>(tile + (off + 64u * j)) : f32x4{};
   }
   __device__ __forceinline__ void product(f32x4 (&acc)[4], const RowFrag<float, D> (&qf)[4]) const {
     for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -281,37 +270,45 @@ template <int D> struct KQuarter<float, D> {
   }
 };
 
+// The sweeps' LDS rings (16-bit inputs, hd = D): slots of 16 keys x 64
+// dimensions (2 KiB) per wave.  Sweep 1 has the whole area below tkey to
+// itself (four tiles in flight); the later sweeps' ring lies beside the
+// candidate lists: two slots at d = 64, where a third would cost a resident
+// block, three at 128.
+constexpr int kSlotBytes = 2048;
+constexpr int ring1_slots(int D) { return 4 * D / 64; }
+constexpr int ring2_slots(int D) { return D == 64 ? 2 : 3; }
+
 // LDS layout, shared by the kernel and the host-side size query.  The class
 // maxima exchanged between the sweeps share their bytes with the candidate
 // lists (they are read before the first candidate is written).
 struct SelLayout {
-  int cand, cm, scm, scr, tk, tkey, drop, fl, cnt, ctl, bits, vlist, total;
+  int cand, cm, scm, ring, tk, tkey, drop, fl, cnt, ctl, bits, vlist, total;
 };
 __host__ __device__ inline int align_up(int x, int a) { return (x + a - 1) / a * a; }
-// Class sets per (row, position) of sweep 1: 4 tighten the sweep-2 floor
-// (fewer candidates) but double the class-maxima exchange in LDS; up to
-// k = 64 the exchange at 2 sets keeps two select blocks per compute unit
-// (at d = 128, k = 64: 68 KB of LDS and 199 VGPRs against 86 KB and 257
-// for 4 sets, measured 11.8 against 17.4 ms at the c4 shape).
-__host__ __device__ inline int classes_per_lane(int k) { return k <= 64 ? 2 : 4; }
-// Sweep-2 value scratch: 16 floats per lane, the lane's 16-byte chunk j
-// stored at chunk j ^ ((lane >> 1) & 3), so that the 8 lanes a 16-byte
-// store serves per cycle hit distinct banks.
-constexpr int kScrStride = 16;
-__host__ __device__ inline SelLayout sel_layout(int k, int cap, int nKB) {
+// Class sets per (row, position) of sweep 1, over NW waves: 64 of 16 NW R
+// classes.  256 classes tighten the sweep-2 floor (fewer candidates) but
+// double the class-maxima exchange in LDS; up to k = 64 the exchange at 128
+// keeps two select blocks per compute unit (at d = 128, k = 64: 68 KB of
+// LDS and 199 VGPRs against 86 KB and 257, measured 11.8 against 17.4 ms
+// over 1x32x16384).
+__host__ __device__ inline int classes_per_lane(int k, int NW) { return (k <= 64 ? 8 : 16) / NW; }
+// ringD: the rings' D, or 0 for the variants without rings.
+__host__ __device__ inline SelLayout sel_layout(int k, int cap, int nKB, int NW, int ringD) {
   SelLayout l;
-  const int R = classes_per_lane(k);
-  l.scm = 64 * R + 4;  // floats per row of the class-maxima exchange (+4: rows 4 banks apart)
-  const int cand_bytes = kBlock * cap * 8;
+  l.scm = 16 * NW * classes_per_lane(k, NW) + 4;  // floats per row of the class-maxima exchange (+4: rows 4 banks apart)
+  const int cand_bytes = kBlock * (cap + 1) * 8;  // rows of cap + 1 slots (see cslot)
   const int cm_bytes = kBlock * l.scm * 4;
-  const int scr_bytes = kThreads * kScrStride * 4;
+  const int ring_bytes = ringD ? NW * ring2_slots(ringD) * kSlotBytes : 0;
   const int tk_bytes = k * kBlock * 4;
   l.cand = 0;
   l.cm = 0;
-  // the value scratch (sweeps) and the sorted top-k values (emission) share bytes
-  l.scr = align_up(cand_bytes > cm_bytes ? cand_bytes : cm_bytes, 16);
-  l.tk = l.scr;
-  l.tkey = l.scr + align_up(scr_bytes > tk_bytes ? scr_bytes : tk_bytes, 16);
+  // the later sweeps' ring and the sorted top-k values (emission) share bytes
+  l.ring = align_up(cand_bytes > cm_bytes ? cand_bytes : cm_bytes, 16);
+  l.tk = l.ring;
+  l.tkey = l.ring + align_up(ring_bytes > tk_bytes ? ring_bytes : tk_bytes, 16);
+  const int ring1_bytes = ringD ? NW * ring1_slots(ringD) * kSlotBytes : 0;
+  if (l.tkey < ring1_bytes) l.tkey = ring1_bytes;
   l.drop = l.tkey + kBlock * 8;
   l.fl = l.drop + kBlock * 8;
   l.cnt = l.fl + kBlock * 4;
@@ -331,31 +328,29 @@ __host__ __device__ inline int select_round_bound(int NK, int k, int cap) {
   return 2 + (NK > cap ? (NK - cap) / (cap - k) + 1 : 0);
 }
 
-// Score pass of one (batch, head) and 64-row query block; 4 waves.  Wave w
-// multiplies its quarter of every visible key tile with all 64 rows (no LDS
-// staging, no barrier inside a sweep); lane (c, g) sees rows 16 cb + c and
-// keys 16 w + 4 g + r of each tile.  R class maxima per (lane, row, r)
-// give 64 R classes per row.
-// Waves per SIMD the headline variant (bf16, d = 64, two classes per lane)
-// is held to: three blocks of its ~50 KB of LDS fit a CU, and 168 VGPRs
-// let three waves share a SIMD (one more VGPR would drop it to two).
-// Sweep 1's LDS ring (16-bit inputs): tiles in flight per wave, and its
-// bytes (four waves x tiles x 16 keys x D x 2 bytes).  It fits below
-// sel_layout's tkey for every k: the class-maxima exchange alone takes
-// 64 (64 R + 4) floats, and the value scratch 16 KiB after it.
-template <int D, int R>
-constexpr int ring_tiles() { return (D == 128 && R == 2) ? 3 : 4; }
-template <int D, int R>
-constexpr int ring_bytes() { return 4 * ring_tiles<D, R>() * 32 * D; }
-
-template <typename T, int D, int R>
-constexpr int select_waves_per_simd() { return sizeof(T) == 2 && D == 64 && R == 2 ? 3 : 1; }
+// Score pass of one (batch, head) and 64-row query block; NW = 4 or 8
+// waves.  Wave w multiplies quarter w % 4 of the visible key tiles it takes
+// (every tile of the list with 4 waves, every other one, from w / 4, with
+// 8) with all 64 rows (no LDS staging, no barrier inside a sweep); lane
+// (c, g) sees rows 16 cb + c and keys 16 (w % 4) + 4 g + r of each tile.  R
+// class maxima per (lane, row, r) give 16 NW R classes per row.
+//
+// Waves per SIMD: three for the headline variant (bf16, d = 64, two classes
+// per lane), whose ~50 KB of LDS let three blocks into a compute unit, and
+// 168 VGPRs three waves onto a SIMD (one more VGPR would drop it to two);
+// two for the 8-wave block.
+template <typename T, int D, int R, int NW>
+constexpr int select_waves_per_simd() { return NW == 8 ? 2 : sizeof(T) == 2 && D == 64 && R == 2 ? 3 : 1; }
 
 // KL: the K layout (KLayout).  With hd = D (kKDense, kKRows) there are no
 // column tests, and with 16-bit inputs sweep 1 reads K through the LDS ring
 // (whose loads read whole rows).
-template <typename T, int D, int MODE, int R, int KL>
-__global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void select_kernel(SelectParams p) {
+template <typename T, int D, int MODE, int R, int KL, int NW>
+__global__ __launch_bounds__(NW * kWave, (select_waves_per_simd<T, D, R, NW>())) void select_kernel(SelectParams p) {
+  static_assert(NW == 4 || NW == 8, "waves per block");
+  constexpr int kThreads = NW * kWave;
+  constexpr int kPhases = NW / 4;     // tiles of the list taken side by side
+  constexpr int kRows = kBlock / NW;  // rows per wave outside the sweeps
   constexpr bool kExact = MODE != kRawDots;
   constexpr bool kTiles = MODE != kGivenScores;
   constexpr int UR = R > 2 ? R : 2;  // sweep-1 unroll: class of a tile = ordinal % R
@@ -363,7 +358,7 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
   const int k = p.d.k, NQ = p.d.NQ, NK = p.d.NK, nKB = p.d.nKB, nQB = p.d.nQB;
   const int cap = p.cap;
   const int nbw = (nKB + 31) >> 5;
-  const SelLayout lay = sel_layout(k, cap, nKB);
+  const SelLayout lay = sel_layout(k, cap, nKB, NW, is_half<T> && KL != kKGeneral ? D : 0);
   uint64_t* s_cand = reinterpret_cast<uint64_t*>(smem + lay.cand);
   float* s_cm = reinterpret_cast<float*>(smem + lay.cm);
   float* s_tk = reinterpret_cast<float*>(smem + lay.tk);
@@ -374,14 +369,14 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
   uint32_t* s_ctl = reinterpret_cast<uint32_t*>(smem + lay.ctl);
   uint32_t* s_bits = reinterpret_cast<uint32_t*>(smem + lay.bits);
   int32_t* s_vlist = reinterpret_cast<int32_t*>(smem + lay.vlist);
-  // Slot of candidate e of row r: rows XOR-ed with bits 3-5 of e (moved to
-  // row bits 1-3), so that the 8 lanes reading entries e = 8i + pp of one
-  // row, and the lanes of two adjacent rows, fall in 16 distinct 8-byte banks.
-  auto cslot = [](int e, int r) { return e * kBlock + (r ^ (((e >> 3) & 7) << 1)); };
+  // Slot of candidate e of row r, rows cap + 1 slots apart: an append's
+  // address is one multiply-add (XOR-ing row bits into a slot-major layout
+  // spread the sort's reads over more banks but cost every append four
+  // more instructions).
+  const int cstride = cap + 1;
+  auto cslot = [&](int e, int r) { return r * cstride + e; };
 
   const int t = threadIdx.x, w = t >> 6, L = t & 63, g = L >> 4, c = L & 15;
-  float* s_scr = reinterpret_cast<float*>(smem + lay.scr) + t * kScrStride;  // this lane's
-  const int scr_sw = ((L >> 1) & 3) << 2;  // chunk swizzle, in floats
   int brank, bh;
   xcd_rank_order(blockIdx.x, nQB, p.d.BH, brank, bh);
   const int qb = nQB - 1 - brank, q0 = qb * kBlock;  // heaviest first
@@ -430,7 +425,10 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
     if (L == 0) s_ctl[1] = uint32_t(n);
   }
   __syncthreads();
-  const int nvis = int(s_ctl[1]);
+  // this wave's tiles of the list: entries phase, phase + kPhases, ...
+  const int phase = kPhases == 1 ? 0 : __builtin_amdgcn_readfirstlane(w >> 2);
+  const int nvis = (int(s_ctl[1]) + kPhases - 1 - phase) / kPhases;
+  const int wq = w & 3;  // and its quarter of them
 
   RowFrag<T, D> qf[4];  // Q^T operands: row 16 cb + c in column c of the products
   const T* Kb = nullptr;
@@ -440,20 +438,41 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
       qf[cb].load(Qh + size_t(rowok[cb] ? q0 + 16 * cb + c : 0) * p.lq.sn, rowok[cb], L, p.d.hd);
     Kb = static_cast<const T*>(p.k) + head_at(p.lk, bh, p.d.H);
   }
-  const uint32_t ksnb = uint32_t(p.lk.sn) * uint32_t(sizeof(T));  // K row stride, bytes (GENERAL loads)
-  const int kq0 = 16 * w + c;  // the lane's A-operand key within a tile
+  // K addressing: a tile's first row from scalar registers plus a 32-bit
+  // lane offset (one load form for every tile; forming 64-bit lane addresses
+  // per step took a quarter of sweep 1's VALU instructions).  Keys >= NK of
+  // the last tile read its last valid key instead: they lie in a partially
+  // visible tile, where the visibility test discards their scores.
+  const uint32_t ksnb = KL == kKDense ? uint32_t(D * sizeof(T)) : uint32_t(p.lk.sn) * uint32_t(sizeof(T));
+  const unsigned char* const Kbytes = reinterpret_cast<const unsigned char*>(Kb);
+  const int klast = NK - 1 - (nKB - 1) * kBlock;  // last valid key of the last tile
+  auto tile_at = [&](int kt) { return Kbytes + size_t(uint32_t(kt)) * (size_t(kBlock) * ksnb); };
+  const int kq0 = 16 * wq + c;  // the lane's A-operand key within a tile
+  const uint32_t koff = uint32_t(kq0) * ksnb + 16u * g, koff_last = uint32_t(min(kq0, klast)) * ksnb + 16u * g;
 
   // One pass over the visible key blocks: body(u, kt, visb, acc) for each,
-  // u = (ordinal of the block) % U known at compile time.  The K quarters of
+  // u = (ordinal of the block in the wave's list) % U known at compile time.  The K quarters of
   // the next two tiles are in flight while a tile is used.  In partially
-  // visible tiles bit 15 - (4 cb + r) of visb is cleared and acc set to
-  // -inf where key 16 w + 4 g + r is not visible to row 16 cb + c (visb is
+  // visible tiles bit 4 cb + r of visb is cleared and acc set to
+  // -inf where key 16 wq + 4 g + r is not visible to row 16 cb + c (visb is
   // 0xffff for a whole tile); the body is called once, after the masking,
-  // so its code is not repeated per case.  The first 64 list entries are
-  // held one per lane.
-  const int vl0 = L < nvis ? s_vlist[L] : 0;
-  auto entry = [&](int i) {
-    return i < kWave ? __builtin_amdgcn_readlane(vl0, i) : __builtin_amdgcn_readfirstlane(s_vlist[i]);
+  // so its code is not repeated per case.  The wave's list entries are held
+  // one per lane, 128 at a time: window() before step i0 (a multiple of 64
+  // or the first) loads entries i0 .. i0 + 127, and entry(i) reads one of
+  // them (reading entries past the first 64 from LDS at each step instead
+  // put two LDS round trips into every step of a long list).
+  int vl[2], vbase = 0;
+  auto list_at = [&](int i) { return i < nvis ? s_vlist[kPhases * i + phase] : 0; };
+  auto window = [&](int i0) {
+    vl[0] = i0 == 0 ? list_at(L) : vl[1];
+    vl[1] = list_at(i0 + kWave + L);
+    vbase = i0;
+  };
+  auto entry = [&](int i) {  // vbase <= i < vbase + 128
+    const int at = i - vbase;
+    const int a0 = __builtin_amdgcn_readlane(vl[0], at & (kWave - 1));
+    const int a1 = __builtin_amdgcn_readlane(vl[1], at & (kWave - 1));
+    return at < kWave ? a0 : a1;
   };
   // Per tile, after its scores are formed: the visibility masking, then
   // body(u, kb0, visb, acc).  The padding of the last group of U tiles
@@ -461,7 +480,7 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
   // tiles' path: a separate path that set acc to constants made the
   // compiler copy acc between register sets on every whole tile.
   auto finish = [&](auto uc, int i, int e, f32x4(&acc)[4], auto&& body) __attribute__((always_inline)) {
-    const int kb0 = (e & 0xffffff) * kBlock + 16 * w + 4 * g;  // the lane's first key
+    const int kb0 = (e & 0xffffff) * kBlock + 16 * wq + 4 * g;  // the lane's first key
     if constexpr (MODE == kExactScores)
       for (int cb = 0; cb < 4; ++cb)
         for (int r = 0; r < 4; ++r) acc[cb][r] = clamp_score(acc[cb][r] * scale);
@@ -473,7 +492,7 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
         const int kp = key < klim ? kidx[key] : INT_MAX;
         for (int cb = 0; cb < 4; ++cb)
           if (!(key < klim && kp <= qpos[cb])) {
-            visb &= ~(1u << (15 - (4 * cb + r)));
+            visb &= ~(1u << (4 * cb + r));
             acc[cb][r] = -__builtin_inff();
           }
       }
@@ -482,10 +501,12 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
   };
   auto sweep = [&](auto u_tag, auto&& body) {
     constexpr int U = decltype(u_tag)::value;
-    if (nvis == 0) return;  // block-uniform
+    if (nvis == 0) return;  // wave-uniform
+    window(0);
     KQuarter<T, D> kq[2];
     auto fetch = [&](KQuarter<T, D>& f, int e) {
-      f.template load<KL>(Kb, (e & 0xffffff) * kBlock + kq0, NK, ksnb, p.d.hd, g);
+      const int kt = e & 0xffffff;
+      f.template load<KL>(tile_at(kt), kt == nKB - 1 ? koff_last : koff, p.d.hd, g);
     };
     // The loads are unconditional (past the end of the list they repeat its
     // last tile), so the number in flight is the same on every path and the
@@ -501,12 +522,13 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
     }
     if constexpr (MODE == kGivenScores) {
       for (int i0 = 0; i0 < nvis; i0 += U) {
+        if (i0 - vbase >= kWave) window(vbase + kWave);
         static_for<0, U>([&](auto uc) {
           constexpr int u = decltype(uc)::value;
           const int i = i0 + u;
           const int e = ent[u & 1];
           f32x4 acc[4];
-          const int kb0 = (e & 0xffffff) * kBlock + 16 * w + 4 * g;
+          const int kb0 = (e & 0xffffff) * kBlock + 16 * wq + 4 * g;
           for (int cb = 0; cb < 4; ++cb)
             for (int r = 0; r < 4; ++r) {
               const int key = kb0 + r;
@@ -531,6 +553,7 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
       ent[0] = entry(2 < nvis ? 2 : nvis - 1);
       fetch(kq[0], ent[0]);
       for (int i0 = 0; i0 < nvis; i0 += U) {
+        if (i0 - vbase >= kWave) window(vbase + kWave);
         static_for<0, U>([&](auto uc) {
           constexpr int u = decltype(uc)::value;
           const int i = i0 + u;
@@ -538,84 +561,115 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
           kq[(u + 1) & 1].product(accs[(u + 1) & 1], qf);
           ent[(u + 1) & 1] = entry(i + 3 < nvis ? i + 3 : nvis - 1);
           fetch(kq[(u + 1) & 1], ent[(u + 1) & 1]);
-          finish(uc, i, ecur, accs[u & 1], body);
+          if (u == 0 || i < nvis) finish(uc, i, ecur, accs[u & 1], body);  // wave-uniform
           ecur = enext;
         });
       }
     }
   };
-  // Sweep 1 (16-bit inputs) reads its K quarters through a ring in LDS
-  // filled by global_load_lds (the loads in flight hold no VGPRs, so each
-  // wave keeps kRing tiles in flight instead of two).  The ring occupies
-  // the candidate lists' and value scratch's bytes, which sweep 1 leaves
-  // unused; each wave owns kRing slots of one wave quarter (16 keys x D
-  // bytes of 2-byte elements, row-major).  The quarter's rows are
-  // contiguous in memory, and each DMA instruction reads whole rows (8 rows
-  // of 128 bytes at D = 64, 4 of 256 at D = 128): a load of 16 half rows,
-  // the MFMA operand layout, streams from L2 at about a third of the rate
-  // (measured at the headline shape: 8.5 against 28 TB/s).  global_load_lds
+  // With 16-bit inputs and hd = D the sweeps read their K quarters through a
+  // ring in LDS filled by global_load_lds (the loads in flight hold no
+  // VGPRs).  Each wave owns NS slots of 16 keys x 64 dimensions, row-major;
+  // a tile takes D / 64 of them.  Each DMA instruction reads 8 rows of 128
+  // contiguous bytes: a load of 16 half rows, the MFMA operand layout,
+  // streams from L2 at a third of the rate (measured at the headline shape:
+  // 8.5 against 28 TB/s), and with it the second sweep ran at that rate
+  // whatever its candidates cost (2150 against 820 clocks per tile and wave
+  // for the first one at d = 128, two waves per SIMD).  global_load_lds
   // puts lane L's 16 bytes at the instruction's base + 16 L, so lane L
   // fetches the chunk that belongs at that place: row r's chunk x is stored
-  // at chunk x ^ sw(r), which makes the operand reads (16 rows at one chunk
-  // per 16 lanes) fall in distinct banks.  The compiler does not order LDS
-  // reads after the DMA that fills them, so the waits are explicit: vmcnt
-  // before a slot is read (the (kRing - 1) younger tiles' loads may stay in
-  // flight), lgkmcnt(0) before a slot is refilled.
-  constexpr int kCh = D / 32;              // DMA instructions (and MFMA k steps) per quarter
-  constexpr int kSlot = kWave * 16 * kCh;  // bytes per wave and tile
-  constexpr int kCpr = D / 8;              // 16-byte chunks per row
-  constexpr int kRpi = kWave / kCpr;       // rows per DMA instruction
-  auto qsw = [](int r) { return D == 64 ? (r >> 1) & 7 : r & 15; };
-  constexpr int kRing = ring_tiles<D, R>();
+  // at chunk x ^ ((r >> 1) & 7), which makes the operand reads (16 rows at
+  // one chunk per 16 lanes) fall in distinct banks.  The compiler does not
+  // order LDS reads after the DMA that fills them, so the waits are
+  // explicit: vmcnt before a slot is read (the (NS - 1) younger slots' loads
+  // may stay in flight), lgkmcnt(0) before a slot is refilled.
   constexpr bool kRingSweep = kTiles && is_half<T> && KL != kKGeneral;
-  auto sweep_ring = [&](auto u_tag, auto&& body) {
-    constexpr int U = decltype(u_tag)::value;
-    if (nvis == 0) return;  // block-uniform
-    unsigned char* ringw = smem + w * kRing * kSlot;  // this wave's slots
-    // lane L of instruction j: quarter row r = kRpi j + L / kCpr, stored
-    // chunk L % kCpr, fetched chunk (L % kCpr) ^ sw(r)
-    auto dma = [&](int slot, int e) __attribute__((always_inline)) {
-      const int kq = (e & 0xffffff) * kBlock + 16 * w;  // the quarter's first key
-      unsigned char* dst = ringw + slot * kSlot;
-      for (int j = 0; j < kCh; ++j) {
-        const int r = kRpi * j + L / kCpr, key = kq + r;
-        const int kk = key < NK ? key : 0, ch = (L % kCpr) ^ qsw(r);
-        const void* src;
-        if constexpr (KL == kKDense)
-          src = Kb + size_t(kk) * D + 8 * ch;
-        else
-          src = reinterpret_cast<const unsigned char*>(Kb) + (uint32_t(kk) * ksnb + 16u * ch);
-        __builtin_amdgcn_global_load_lds(src,
-                                         (__attribute__((address_space(3))) void*)(dst + j * kWave * 16),
-                                         16, 0, 0);
-      }
+  auto sweep_ring = [&](auto ns_tag, int ring_at, auto&& body) {
+   if constexpr (kRingSweep) {
+    constexpr int NS = decltype(ns_tag)::value;
+    constexpr int KH = D / 64;                           // slots per tile
+    constexpr int UT = NS % KH == 0 ? NS / KH : NS;      // tiles after which the slots repeat
+    if (nvis == 0) return;  // wave-uniform
+    window(0);
+    unsigned char* ringw = smem + ring_at + __builtin_amdgcn_readfirstlane(w) * NS * kSlotBytes;
+    // lane L of instruction j: quarter row r = 8 j + L / 8, stored chunk
+    // L % 8, fetched chunk (L % 8) ^ ((r >> 1) & 7)
+    uint32_t doff[2], doff_last[2], roff[2];
+    for (int j = 0; j < 2; ++j) {
+      const int r = 8 * j + L / 8, key = 16 * wq + r;
+      const uint32_t ch = 16u * uint32_t((L % 8) ^ ((r >> 1) & 7));
+      doff[j] = uint32_t(key) * ksnb + ch;
+      doff_last[j] = uint32_t(min(key, klast)) * ksnb + ch;
+      // operand j of lane (c, g): quarter row c, chunk 4 j + g
+      roff[j] = uint32_t(c * 128 + 16 * ((4 * j + g) ^ ((c >> 1) & 7)));
+    }
+    auto dma = [&](int slot, int e, int half) __attribute__((always_inline)) {
+      const int kt = e & 0xffffff;
+      const unsigned char* tile = tile_at(kt) + 128 * half;
+      const bool last = kt == nKB - 1;
+      for (int j = 0; j < 2; ++j)
+        lds_dma16(tile + (last ? doff_last[j] : doff[j]), ringw + slot * kSlotBytes + j * kWave * 16);
     };
     // The Q fragments' loads are waited for here, by an s_waitcnt the
     // compiler sees: otherwise its wait for them before the first product
     // stays in the loop as vmcnt(0) on every tile (encoding: vmcnt 0,
     // expcnt 7, lgkmcnt 15).
     __builtin_amdgcn_s_waitcnt(0x0f70);
-    for (int j = 0; j < kRing; ++j) dma(j, entry(j < nvis ? j : nvis - 1));
-    int slot = 0;  // slot of tile i
-    for (int i0 = 0; i0 < nvis; i0 += U) {
-      static_for<0, U>([&](auto uc) {
-        const int i = i0 + decltype(uc)::value;
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kRing - 1) * kCh) : "memory");
-        KQuarter<T, D> kq;
-        using A = std::remove_reference_t<decltype(kq.a[0])>;
-        // operand s of lane (c, g): quarter row c, chunk 4 s + g
-        for (int s = 0; s < kCh; ++s)
-          kq.a[s] = *reinterpret_cast<const A*>(ringw + slot * kSlot + c * (16 * kCpr) +
-                                                16 * ((4 * s + g) ^ qsw(c)));
-        f32x4 acc[4];
-        kq.product(acc, qf);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        dma(slot, entry(i + kRing < nvis ? i + kRing : nvis - 1));
-        slot = slot + 1 == kRing ? 0 : slot + 1;
-        finish(uc, i, entry(i < nvis ? i : nvis - 1), acc, body);
-      });
+    for (int q = 0; q < NS; ++q) dma(q, entry(min(q / KH, nvis - 1)), q % KH);
+    for (int i0 = 0; i0 < nvis; i0 += UT) {
+      if (i0 - vbase >= kWave) window(vbase + kWave);
+      if constexpr (KH == 1) {
+        // d = 64: two tiles per step, so that a step's latencies (operand
+        // reads, products, their results) are paid once for both
+        static_for<0, UT / 2>([&](auto uc) {
+          constexpr int u = 2 * decltype(uc)::value;
+          const int i = i0 + u;
+          if (i >= nvis) return;  // wave-uniform
+          using V8 = typename Half<T>::v8;
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * 2) : "memory");
+          V8 a[2][2];
+          for (int q = 0; q < 2; ++q)
+            for (int j = 0; j < 2; ++j)
+              a[q][j] = *reinterpret_cast<const V8*>(ringw + (u + q) * kSlotBytes + roff[j]);
+          f32x4 acc[2][4];
+          for (int q = 0; q < 2; ++q)
+            for (int cb = 3; cb >= 0; --cb) acc[q][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+          // KQuarter's products: reduction steps in order
+          for (int j = 0; j < 2; ++j)
+            for (int q = 0; q < 2; ++q)
+              for (int cb = 3; cb >= 0; --cb) acc[q][cb] = mfma(a[q][j], qf[cb].v[j], acc[q][cb]);
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          for (int q = 0; q < 2; ++q) dma(u + q, entry(min(i + q + NS, nvis - 1)), 0);
+          finish(std::integral_constant<int, u>{}, i, entry(i), acc[0], body);
+          if (i + 1 < nvis)  // wave-uniform
+            finish(std::integral_constant<int, u + 1>{}, i + 1, entry(i + 1), acc[1], body);
+        });
+      } else {
+        static_for<0, UT>([&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          const int i = i0 + u;
+          if (i >= nvis) return;  // wave-uniform
+          using V8 = typename Half<T>::v8;
+          f32x4 acc[4];
+          for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+          static_for<0, KH>([&](auto hc) {
+            constexpr int h = decltype(hc)::value, slot = (u * KH + h) % NS;
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * 2) : "memory");
+            V8 a[2];
+            for (int j = 0; j < 2; ++j)
+              a[j] = *reinterpret_cast<const V8*>(ringw + slot * kSlotBytes + roff[j]);
+            // KQuarter's products: reduction steps s = 2 h + j in order
+            for (int j = 0; j < 2; ++j)
+              for (int cb = 3; cb >= 0; --cb) acc[cb] = mfma(a[j], qf[cb].v[2 * h + j], acc[cb]);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            dma(slot, entry(min(i + (h + NS) / KH, nvis - 1)), (h + NS) % KH);
+          });
+          finish(uc, i, entry(i), acc, body);
+        });
+      }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+   }
   };
 
   // ---------------- sweep 1: class maxima ----------------
@@ -629,25 +683,26 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
       for (int r = 0; r < 4; ++r) cm[cb][r + 4 * j] = vmax(cm[cb][r + 4 * j], acc[cb][r], pinf);
   };
   if constexpr (kRingSweep) {
-    sweep_ring(std::integral_constant<int, UR>{}, maxima);
+    sweep_ring(std::integral_constant<int, ring1_slots(D)>{}, 0, maxima);
     __syncthreads();  // every wave's ring reads are done before the exchange reuses the bytes
   } else {
     sweep(std::integral_constant<int, UR>{}, maxima);
   }
 
-  // Exchange: row 16 cb + c's 64 R class maxima, 4 R from each of its 16
-  // lanes (4 waves x 4 lane groups), then wave w finds the floors of rows
-  // 16 w + c, lane group g holding classes [16 R g, 16 R (g + 1)).
+  // Exchange: row 16 cb + c's 16 NW R class maxima, 4 R from each of its
+  // 4 NW lanes (NW waves x 4 lane groups), then wave w finds the floors of
+  // rows kRows w + L % kRows, the row's lane L / kRows holding classes
+  // [16 R (L / kRows), 16 R (L / kRows + 1)).
   for (int cb = 0; cb < 4; ++cb)
     for (int r = 0; r < 4; ++r)
       for (int j = 0; j < R; ++j)
         s_cm[(16 * cb + c) * lay.scm + ((w * 4 + g) * 4 + r) * R + j] = cm[cb][r + 4 * j];
   __syncthreads();
   {
-    const int row = 16 * w + c;
+    const int row = kRows * w + L % kRows, part = L / kRows;
     float v[16 * R];
     for (int i = 0; i < 16 * R; i += 4) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(s_cm + row * lay.scm + 16 * R * g + i);
+      const f32x4 x = *reinterpret_cast<const f32x4*>(s_cm + row * lay.scm + 16 * R * part + i);
       for (int j = 0; j < 4; ++j) v[i + j] = x[j];
     }
     // a value x with at least k class maxima >= x (bisection between the
@@ -661,23 +716,41 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
         hi = fmaxf(hi, v[i]);
       }
     }
-    const int nf = group_sum(int(nfin));
-    lo = group_min(lo);
-    hi = group_max(hi);
+    const int nf = row_sum<NW>(int(nfin));
+    lo = row_min<NW>(lo);
+    hi = row_max<NW>(hi);
     float x = -__builtin_inff();
-    if (nf >= k) {
-      for (int it = 0; it < 8; ++it) {
-        const float mid = 0.5f * (lo + hi);
-        uint32_t cnt = 0;
-        for (int i = 0; i < 16 * R; ++i) cnt = count_ge(cnt, v[i], mid);
-        if (group_sum(int(cnt)) >= k) lo = mid;
-        else hi = mid;
-      }
-      x = lo;
+    auto at_least = [&](float m) {  // class maxima of the row >= m
+      uint32_t cnt = 0;
+      for (int i = 0; i < 16 * R; ++i) cnt = count_ge(cnt, v[i], m);
+      return row_sum<NW>(int(cnt));
+    };
+    for (int it = 0; it < 8; ++it) {
+      const float mid = 0.5f * (lo + hi);
+      if (at_least(mid) >= k) lo = mid;
+      else hi = mid;
     }
+    // Eight steps are enough where a row's maxima spread evenly.  Where they
+    // fall into clumps (clustered keys) lo can still be below many of them,
+    // and lists of 1.75 k then overflow (a third sweep on most blocks at
+    // 1x32x16384, k = 64): more steps until k + k / 32 at most reach lo.
+    if (k > 42) {  // block-uniform; below, the lists hold k + 32
+      int nlo = at_least(lo);
+      for (int it = 0; it < 16 && __any(nlo > k + (k >> 5)); ++it) {
+        const float mid = 0.5f * (lo + hi);
+        const int n = at_least(mid);
+        if (n >= k) {
+          lo = mid;
+          nlo = n;
+        } else {
+          hi = mid;
+        }
+      }
+    }
+    if (nf >= k) x = lo;
     const float th = kExact ? x : (x == -__builtin_inff() ? x : clamp_score(x * scale));
     // NaN marks a row that collects nothing (past NQ)
-    if (g == 0) s_fl[row] = q0 + row < NQ ? sweep_floor(th, kExact, scale) : __builtin_nanf("");
+    if (part == 0) s_fl[row] = q0 + row < NQ ? sweep_floor(th, kExact, scale) : __builtin_nanf("");
   }
   __syncthreads();
 
@@ -705,56 +778,60 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
     for (int cb = 0; cb < 4; ++cb) {
       fl[cb] = s_fl[16 * cb + c];
       if (fl[cb] == 0.0f) fl[cb] = -0.0f;
-      if (!__builtin_isnan(fl[cb])) cmask |= 0xfu << (12 - 4 * cb);  // bit order of collect's m
-      if (fl[cb] == -__builtin_inff()) amask |= 0xfu << (12 - 4 * cb);
+      if (!__builtin_isnan(fl[cb])) cmask |= 0xfu << (4 * cb);  // bit order of collect's m
+      if (fl[cb] == -__builtin_inff()) amask |= 0xfu << (4 * cb);
     }
     // Candidates are stored raw, (index << 32) | bits of the sweep value,
     // and turned into selection keys when they are sorted.  Per tile, the
-    // lane's candidate bits m (bit 15 - (4 cb + r): key kb0 + r of row
+    // lane's candidate bits m (bit 4 cb + r: key kb0 + r of row
     // 16 cb + c) come branch-free, two instructions per score, in the order
-    // the MFMA results arrive (cb = 0 first); the few lanes with
-    // candidates then park their 16 values in their LDS scratch and append
-    // one candidate per round (LDS atomic on the row's count), so the wave
-    // runs as many rounds as its busiest lane has candidates (about two at
-    // the headline shape) instead of visiting every slot.  (Storing every
-    // candidate straight from its register instead, one atomic per row and
-    // 16 predicated stores, measured 1.5 times slower: the predicated
-    // stores cost more VALU than the LDS round trips they remove.)
+    // the MFMA results arrive (cb = 0 first); the few lanes with candidates
+    // then append two per trip (LDS atomics on the rows' counts), so the
+    // wave runs half as many trips as its busiest lane has candidates.
     auto collect = [&](int kb0, uint32_t visb, f32x4 (&acc)[4], auto later) {
-      // bit 15 - (4 cb + r) <- sign of v - fl: set where v < fl, so that
+      // bit 4 cb + r <- sign of v - fl: set where v < fl, so that
       // the complement marks !(v < fl) (NaN differences have a clear sign
       // bit)
       uint32_t m = 0;
-      for (int cb = 0; cb < 4; ++cb)
-        for (int r = 0; r < 4; ++r)
+      for (int cb = 3; cb >= 0; --cb)
+        for (int r = 3; r >= 0; --r)
           m = __builtin_amdgcn_alignbit(m, __float_as_uint(acc[cb][r] - fl[cb]), 31);
       m = (~m | amask) & cmask & visb;
-      if (m != 0u) {
-        for (int cb = 0; cb < 4; ++cb) *reinterpret_cast<f32x4*>(s_scr + ((4 * cb) ^ scr_sw)) = acc[cb];
-      }
-      while (m != 0u) {
-        const int b = 15 - __builtin_ctz(m);  // 4 cb + r
-        m &= m - 1u;
-        const int row = 4 * (b & 12) + c, key = kb0 + (b & 3);
-        const float v = s_scr[b ^ scr_sw];
-        if constexpr (decltype(later)::value) {
-          if (make_key(kExact ? v : clamp_score(v * scale), key) < s_tkey[row]) continue;
+      // score b = 4 cb + r by selects (parking the 16 scores in LDS to read
+      // one back took the bytes that the later sweeps' ring now has)
+      auto pick = [&](int b) {
+        float x[4];
+        for (int r = 0; r < 4; ++r) {
+          const float lo = (b & 4) ? acc[1][r] : acc[0][r], hi = (b & 4) ? acc[3][r] : acc[2][r];
+          x[r] = (b & 8) ? hi : lo;
         }
-        const uint32_t pos = atomicAdd(&s_cnt[row], 1u);
+        const float lo = (b & 1) ? x[1] : x[0], hi = (b & 1) ? x[3] : x[2];
+        return (b & 2) ? hi : lo;
+      };
+      auto append = [&](int row, int key, float v, uint32_t pos) {
         if (pos < uint32_t(cap))
           s_cand[cslot(pos, row)] = (uint64_t(uint32_t(key)) << 32) | __float_as_uint(v);
         else  // the best candidate left out
           atomicMax(&s_drop[row], make_key(kExact ? v : clamp_score(v * scale), key));
+      };
+      while (m != 0u) {
+        const int b = __builtin_ctz(m);  // 4 cb + r
+        m &= m - 1u;
+        const int row = 4 * (b & 12) + c, key = kb0 | (b & 3);
+        const float v = pick(b);
+        if constexpr (decltype(later)::value) {
+          if (make_key(kExact ? v : clamp_score(v * scale), key) < s_tkey[row]) continue;
+        }
+        append(row, key, v, atomicAdd(&s_cnt[row], 1u));
       }
     };
-    if (round == 0)
-      sweep(std::integral_constant<int, 2>{}, [&](auto, int kb0, uint32_t visb, f32x4 (&acc)[4]) {
-        collect(kb0, visb, acc, std::false_type{});
-      });
-    else
-      sweep(std::integral_constant<int, 2>{}, [&](auto, int kb0, uint32_t visb, f32x4 (&acc)[4]) {
-        collect(kb0, visb, acc, std::true_type{});
-      });
+    auto collect_sweep = [&](auto later) {
+      auto body = [&](auto, int kb0, uint32_t visb, f32x4 (&acc)[4]) { collect(kb0, visb, acc, later); };
+      if constexpr (kRingSweep) sweep_ring(std::integral_constant<int, ring2_slots(D)>{}, lay.ring, body);
+      else sweep(std::integral_constant<int, 2>{}, body);
+    };
+    if (round == 0) collect_sweep(std::false_type{});
+    else collect_sweep(std::true_type{});
     __syncthreads();
     max_round = round;
     // Rows that overflowed: with T the k-th best stored key, every top-k key
@@ -762,7 +839,7 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
     // top-k in the list and is done.  That is the rule where many keys tie
     // at the score clamp: the lists fill in nearly ascending key order, so
     // the left-out ties come after the kept ones.  With the larger lists
-    // above k = 42 (select_capacity) a block's overflow rounds fell from two
+    // above k = 42 (select_plan) a block's overflow rounds fell from two
     // to one: clustered keys, 1x32x16384, d = 128, k = 64, 11.3 -> 9.9 ms;
     // 1x8x32768 with 16 heavy keys, d = 128, k = 128, 10.6 -> 4.9 ms.
     // The others take T as an exact threshold, restart their lists, and the
@@ -770,25 +847,30 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
     if (t < kBlock && q0 + t < NQ && s_cnt[t] > uint32_t(cap)) s_ctl[0] = uint32_t(round + 1);
     __syncthreads();
     if (s_ctl[0] != uint32_t(round + 1)) break;  // block-uniform
-    for (int j = 0; j < 16; ++j) {
-      const int r = 16 * w + j;
+    for (int j = 0; j < kRows; ++j) {
+      const int r = kRows * w + j;
       const bool over = q0 + r < NQ && s_cnt[r] > uint32_t(cap);  // wave-uniform
       if (!over) {
         if (L == 0) s_fl[r] = __builtin_nanf("");
         continue;
       }
-      // T by bisection between the smallest and largest stored key (the
-      // keys are distinct: some bound is met by exactly k of them), four
-      // compares and population counts per step
-      uint64_t v[4], lo = ~0ull, hi = 0ull;
+      // T by bisection between bounds of the stored keys (their smallest
+      // and largest score and index words), four compares and population
+      // counts per step; the keys are distinct: some bound is met by exactly
+      // k of them
+      uint64_t v[4];
+      uint32_t hmin = ~0u, hmax = 0u, lmin = ~0u, lmax = 0u;
       for (int e = 0; e < 4; ++e) {
         const bool in = L + kWave * e < cap;
         v[e] = in ? raw_key(s_cand[cslot(L + kWave * e, r)]) : 0ull;
-        lo = in && v[e] < lo ? v[e] : lo;
-        hi = in && v[e] > hi ? v[e] : hi;
+        const uint32_t h = uint32_t(v[e] >> 32), l = uint32_t(v[e]);
+        hmin = in ? min(hmin, h) : hmin;
+        hmax = in ? max(hmax, h) : hmax;
+        lmin = in ? min(lmin, l) : lmin;
+        lmax = in ? max(lmax, l) : lmax;
       }
-      lo = wave_minmax64<false>(lo);
-      hi = wave_minmax64<true>(hi);
+      uint64_t lo = (uint64_t(wave_minmax_u32<false>(hmin)) << 32) | wave_minmax_u32<false>(lmin);
+      uint64_t hi = (uint64_t(wave_minmax_u32<true>(hmax)) << 32) | wave_minmax_u32<true>(lmax);
       while (lo < hi) {  // count(>= lo) >= k; T in [lo, hi]
         const uint64_t mid = hi - ((hi - lo) >> 1);
         int n = 0;
@@ -796,9 +878,12 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
         if (n >= k) lo = mid;
         else hi = mid - 1;
         if (n == k) {  // T is the smallest key >= mid
-          uint64_t m = ~0ull;
-          for (int e = 0; e < 4; ++e) m = v[e] >= mid && v[e] < m ? v[e] : m;
-          lo = hi = wave_minmax64<false>(m);
+          uint32_t h = ~0u, l = ~0u;
+          for (int e = 0; e < 4; ++e) h = v[e] >= mid ? min(h, uint32_t(v[e] >> 32)) : h;
+          h = wave_minmax_u32<false>(h);
+          for (int e = 0; e < 4; ++e)
+            l = v[e] >= mid && uint32_t(v[e] >> 32) == h ? min(l, uint32_t(v[e])) : l;
+          lo = hi = (uint64_t(h) << 32) | wave_minmax_u32<false>(l);
         }
       }
       if (L == 0) {
@@ -829,11 +914,11 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
 
   // ---------------- select: sort each row's candidates ----------------
   // The top-k key blocks go into the mask bitmap of the row's 32-row half
-  // (wave w sorts rows 16 w .. 16 w + 15, half w / 2): with at most 64 key
+  // (wave w sorts rows kRows w .. kRows w + kRows - 1): with at most 64 key
   // blocks as one register word per lane, OR-ed over the wave at the end
   // (the per-entry LDS atomics would all hit the same two words).
   const bool kb_word = nKB <= 64;
-  uint32_t* s_hbits = s_bits + (w >> 1) * nbw;
+  uint32_t* s_hbits = s_bits + (kRows * w / 32) * nbw;
   uint64_t kbm = 0;
   auto emit = [&](int r, int e, uint64_t key) {
     if (e >= k || q0 + r >= NQ) return;
@@ -946,7 +1031,7 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
     }
   };
   const bool want_topk = p.topk_idx != nullptr;
-  for (int base = 16 * w; base < 16 * w + 16; base += 8) {
+  for (int base = kRows * w; base < kRows * (w + 1); base += 8) {
     int need = k;
     for (int j = 0; j < 8; ++j) need = max(need, ncand(base + j));
     if (want_topk) {
@@ -1007,39 +1092,45 @@ __global__ __launch_bounds__(kThreads, (select_waves_per_simd<T, D, R>())) void 
   }
 }
 
-template <typename T, int D, int MODE, int R, int KL>
+template <typename T, int D, int MODE, int R, int KL, int NW>
 hipError_t launch_one(const SelectParams& p, hipStream_t s) {
-  const SelLayout l = sel_layout(p.d.k, p.cap, p.d.nKB);
-  auto kern = select_kernel<T, D, MODE, R, KL>;
-  if (KL != kKGeneral && is_half<T> && MODE != kGivenScores && ring_bytes<D, R>() > l.tkey)
-    return hipErrorInvalidValue;
+  const SelLayout l =
+      sel_layout(p.d.k, p.cap, p.d.nKB, NW, is_half<T> && KL != kKGeneral ? D : 0);
+  auto kern = select_kernel<T, D, MODE, R, KL, NW>;
   if (l.total > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, l.total);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kern, dim3(p.d.nQB * p.d.BH), dim3(kThreads), l.total, s, p);
+  hipLaunchKernelGGL(kern, dim3(p.d.nQB * p.d.BH), dim3(NW * kWave), l.total, s, p);
   return hipGetLastError();
 }
 
 // The hd = D variants (kKDense, kKRows) for the 16-bit MFMA sweeps with raw
-// dots (the usual scale > 0); the others take the general loads (and
-// sweep 1 on the register path).
-template <typename T, int D, int MODE, int R>
+// dots (the usual scale > 0) that read K through the LDS rings; the others
+// take the general loads into registers.
+template <typename T, int D, int MODE, int R, int NW>
 hipError_t launch_ring(const SelectParams& p, hipStream_t s) {
   if constexpr (is_half<T> && MODE == kRawDots)
-    if (p.d.hd == D) {
-      if (p.lk.sn == D) return launch_one<T, D, MODE, R, kKDense>(p, s);
-      return launch_one<T, D, MODE, R, kKRows>(p, s);
+    if (p.ring) {
+      if (p.lk.sn == D) return launch_one<T, D, MODE, R, kKDense, NW>(p, s);
+      return launch_one<T, D, MODE, R, kKRows, NW>(p, s);
     }
-  return launch_one<T, D, MODE, R, kKGeneral>(p, s);
+  return launch_one<T, D, MODE, R, kKGeneral, NW>(p, s);
 }
 
-// Class sets per (row, position): classes_per_lane.
+// Class sets per (row, position): classes_per_lane; waves: select_plan.
 template <typename T, int D, int MODE>
 hipError_t launch_r(const SelectParams& p, hipStream_t s) {
-  if (classes_per_lane(p.d.k) == 2) return launch_ring<T, D, MODE, 2>(p, s);
-  return launch_ring<T, D, MODE, 4>(p, s);
+  if constexpr (MODE == kRawDots)
+    if (p.waves == 8)
+    {
+      if constexpr (is_half<T> && D == 128)
+        if (p.d.k <= 64) return launch_ring<T, D, MODE, 1, 8>(p, s);
+      return launch_ring<T, D, MODE, 2, 8>(p, s);
+    }
+  if (p.d.k <= 64) return launch_ring<T, D, MODE, 2, 4>(p, s);
+  return launch_ring<T, D, MODE, 4, 4>(p, s);
 }
 
 template <typename T, int D>
@@ -1054,7 +1145,6 @@ hipError_t launch_type(const SelectParams& p, hipStream_t s) {
   if (p.d.D == 128) return launch_mode<T, 128>(p, s);
   return hipErrorInvalidValue;
 }
-
 
 }  // namespace
 

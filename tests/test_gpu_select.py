@@ -163,3 +163,40 @@ def test_select_ties_beyond_the_list_bit_exact(dev, k, with_topk):
     st = _run(dev, S, qidx, kidx, k, 1.5, 1, 1, with_topk)
     sel, c = _oracle(S, qidx, kidx, k, 1.5)
     _compare(st, sel, c)
+
+
+@pytest.mark.parametrize("layout", ["dense", "rows"])
+@pytest.mark.parametrize("k", [1, 32, 42, 43, 64, 65, 128])
+@pytest.mark.parametrize("d,dtype", [(64, torch.bfloat16), (128, torch.bfloat16), (128, torch.float16),
+                                     (96, torch.bfloat16), (64, torch.float32), (128, torch.float32)])
+def test_score_pass_variants(dev, d, dtype, k, layout):
+    """Every variant of the score pass (4 or 8 waves per block, LDS rings or
+    register loads, contiguous or strided K) on visible lists of more than
+    128 tiles (two refills of the per-lane list window, an odd number of
+    tiles, a ragged last one) and on short ones: top-k, mask and tau against
+    the oracle, on scores that are exact in fp32."""
+    import splash_attention as sa
+
+    B, H, NQ, NK, scale = 1, 2, 75, 64 * 130 + 5, 0.125
+    print(f"[select] variants d={d} {dtype} k={k} {layout}", flush=True)
+    g = torch.Generator().manual_seed(100 * d + k)
+    Q, K = ((torch.round(torch.randn(B, H, n, d, generator=g) * 16) / 16).clamp(-4, 4)
+            for n in (NQ, NK))
+    K[:, :, 3000:3300] = K[:, :, 5000:5300]  # ties across tiles
+    kidx = causal_idx(B * H, NK)
+    qidx = torch.randint(40, NK, (B * H, NQ), generator=g).to(torch.int32)
+    qidx[:, :64] = qidx[:, :64].clamp(min=64 * 129)  # the first block sees every tile
+    q, kk = Q.to(dtype).to(dev), K.to(dtype).to(dev)
+    if layout == "rows":
+        kk = torch.cat((kk, kk), -1)[..., :d]  # rows 2 d elements apart
+    got = [sa.ops.splash_forward(q, kk, kk, qidx.to(dev), kidx.to(dev), 1.5, k, scale,
+                                 with_topk=t, with_support=False)[1] for t in (True, False)]
+    torch.cuda.synchronize()
+    S, vis = orc.scores(Q.reshape(B * H, NQ, d).numpy(), K.reshape(B * H, NK, d).numpy(),
+                        qidx.numpy(), kidx.numpy(), scale)
+    sel = orc.select(S, vis, k, 1.5)
+    np.testing.assert_array_equal(got[0].topk_idx.cpu().numpy(), sel.topk_idx)
+    np.testing.assert_array_equal(got[0].topk_val.cpu().numpy(), sel.topk_val)
+    for st in got:
+        np.testing.assert_array_equal(st.mask.cpu().numpy(), sel.mask)
+        np.testing.assert_array_equal(st.taus.cpu().numpy(), sel.taus)
