@@ -302,6 +302,75 @@ __device__ __forceinline__ void tile_t_x_acc(f32x4 (&o)[D / 16], const float* rm
     }
 }
 
+// ---------------------------------------------------------------------------
+// fp32 products on the bf16 matrix unit (d <= 64).  x = h + m + l with three
+// bf16 terms of 8 significant bits each is exact for every finite x that is
+// 0 or at least 2^-109, and a product keeps the six terms down to 2^-18 of
+// it: l h', h l', m m', m h', h m', h h' (the three left out are below 2^-25
+// of |x x'|, less than an fp32 multiply-add's rounding).  Six
+// v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
+// v_mfma_f32_16x16x4_f32 take 256.  |x| beyond bf16's largest value is
+// clamped into h, so that m and l carry the rest; an infinity or a NaN makes
+// l a NaN, and every product of it a NaN.  Tiles with a non-finite score or
+// an operand below 2^-109 (split_low) run again with fp32 products.
+// ---------------------------------------------------------------------------
+struct Split8 {
+  bf16x8 h, m, l;
+};
+__device__ __forceinline__ Split8 split8(const f32x4& a, const f32x4& b) {
+  constexpr float kMax = 0x1.fep127f;  // bf16's largest
+  Split8 r;
+  for (int i = 0; i < 8; ++i) {
+    const float x = i < 4 ? a[i & 3] : b[i & 3];
+    r.h[i] = static_cast<__bf16>(__builtin_amdgcn_fmed3f(x, -kMax, kMax));
+    const float x1 = x - static_cast<float>(r.h[i]);
+    r.m[i] = static_cast<__bf16>(x1);
+    r.l[i] = static_cast<__bf16>(x1 - static_cast<float>(r.m[i]));
+  }
+  return r;
+}
+// acc[f] += A[f] . b for N independent accumulators, smallest terms first.
+template <int N>
+__device__ __forceinline__ void mfma_split(f32x4 (&acc)[N], const Split8 (&a)[N], const Split8& b) {
+  for (int f = 0; f < N; ++f) acc[f] = mfma(a[f].l, b.h, acc[f]);
+  for (int f = 0; f < N; ++f) acc[f] = mfma(a[f].h, b.l, acc[f]);
+  for (int f = 0; f < N; ++f) acc[f] = mfma(a[f].m, b.m, acc[f]);
+  for (int f = 0; f < N; ++f) acc[f] = mfma(a[f].m, b.h, acc[f]);
+  for (int f = 0; f < N; ++f) acc[f] = mfma(a[f].h, b.m, acc[f]);
+  for (int f = 0; f < N; ++f) acc[f] = mfma(a[f].h, b.h, acc[f]);
+}
+// Smallest 2 |bits| - 1 of four values (a zero gives the largest code), and
+// whether such a minimum means a nonzero value below 2^-109.
+__device__ __forceinline__ uint32_t split_min(uint32_t m, const f32x4& x) {
+  for (int i = 0; i < 4; ++i) m = min(m, (__float_as_uint(x[i]) << 1) - 1u);
+  return m;
+}
+__device__ __forceinline__ bool split_low(uint32_t m) { return m < ((127u - 109u) << 24) - 1u; }
+// Whether any of the accumulators of the wave is infinite or NaN.
+template <int N>
+__device__ __forceinline__ bool any_nonfinite(const f32x4 (&acc)[N]) {
+  float s = 0.0f;
+  for (int f = 0; f < N; ++f)
+    for (int r = 0; r < 4; ++r) s = fmaf(acc[f][r], 0.0f, s);
+  return __any(s != 0.0f);  // 0 * inf and 0 * NaN are NaN
+}
+// A row as split B operands: term i of reduction step s covers dimensions
+// 32 s + 8 g .. + 7 in lane group g (the bf16 RowFrag's layout).
+template <int D> struct SplitRow {
+  Split8 v[D / 32];
+  uint32_t low;  // split_min of the lane's values
+  __device__ void load(const float* row, bool ok, int lane, int hd = D) {
+    const int g = lane >> 4;
+    low = ~0u;
+    for (int s = 0; s < D / 32; ++s) {
+      const int d0 = 32 * s + 8 * g;
+      const f32x4 a = ok && d0 < hd ? *reinterpret_cast<const f32x4*>(row + d0) : f32x4{};
+      const f32x4 b = ok && d0 + 4 < hd ? *reinterpret_cast<const f32x4*>(row + d0 + 4) : f32x4{};
+      v[s] = split8(a, b);
+      low = split_min(split_min(low, a), b);
+    }
+  }
+};
 // Exponent classes of the per-score powers, chosen from alpha:
 //   p = u^(1/(alpha-1)), w = u^((2-alpha)/(alpha-1)) = p^(2-alpha), and the
 //   tau recurrence's f'' terms u^((3-2 alpha)/(alpha-1)) (class V).

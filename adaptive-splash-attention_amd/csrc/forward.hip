@@ -183,6 +183,255 @@ __global__ __launch_bounds__(kThreads) void forward_kernel(ForwardParams p) {
   }
 }
 
+// fp32 at d <= 64 (split_ok): the one-block kernel on the bf16 matrix unit
+// (asa_tiles.hpp, split products).  K and V tiles are split into their three
+// bf16 planes once, as they are staged (55 KB of LDS for one tile pair: two
+// blocks per compute unit; the next pair loads into registers meanwhile),
+// the weights in registers; the scores and P V then take 96 matrix products
+// per tile and wave at 16 cycles instead of 128 at 32.  The splitting (about
+// 330 VALU instructions per tile and wave) and the planes' LDS reads (48 KB)
+// take about as long as the products.  G = 2: two groups of four waves take
+// every other tile of the list, and the second one's sums are added to the
+// first one's at the end, where the query blocks alone leave compute units
+// with one wave per SIMD.  Measured against forward_kernel: 4x16x4096x64
+// 1249 -> 980 us, 2x8x2048x64 125 -> 102 us, 1x4x4096x64 219 -> 150 us; the
+// output's 2-norm error against float64 falls from 1.2e-6 to 0.8e-6.
+template <int D> struct alignas(16) SplitFwdSmem {
+  u16 K[3][kBlock * Tile<u16, D>::kRs];
+  u16 V[3][kBlock * Tile<u16, D>::kRs];
+  int kid[kBlock];
+  int low[4];  // low[0]: 1 + the last step whose tiles hold a value below 2^-109
+};
+
+template <int D, int PC, bool EMIT, bool HALF, int G>
+__global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_split[];
+  constexpr int kRs = Tile<u16, D>::kRs;
+  using St = Stager<float, D>;
+  const int NQ = p.d.NQ, NK = p.d.NK, nQB = p.d.nQB, nKB = p.d.nKB;
+  const int grp = G == 1 ? 0 : int(threadIdx.x) / kThreads, t = threadIdx.x % kThreads;
+  const int w = t >> 6, lane = t & 63;
+  SplitFwdSmem<D>& sm = reinterpret_cast<SplitFwdSmem<D>*>(smem_split)[grp];
+  const int g = lane >> 4, c16 = lane & 15;
+  int brank, bh;
+  xcd_rank_order(blockIdx.x, nQB, p.d.BH, brank, bh);
+  const int qb = nQB - 1 - brank;  // heaviest first
+  const int q = qb * kBlock + 16 * w + c16;  // this lane's query row
+  const bool qok = q < NQ;
+  const size_t row = size_t(bh) * NQ + (qok ? q : 0);
+  const int H = p.d.H, hd = p.d.hd;
+
+  const float* Kb = static_cast<const float*>(p.k) + head_at(p.lk, bh, H);
+  const float* Vb = static_cast<const float*>(p.v) + head_at(p.lv, bh, H);
+  const int32_t* kidx = p.k_idx + size_t(bh) * NK;
+  const float* qrow = static_cast<const float*>(p.q) + head_at(p.lq, bh, H) + size_t(qok ? q : 0) * p.lq.sn;
+  SplitRow<D> qf;
+  qf.load(qrow, qok, lane, hd);
+  const int qpos = qok ? p.q_idx[row] : 0;
+  const float am1 = p.d.alpha - 1.0f;
+  const float a = 1.0f / am1;
+  const SignedClip clip(am1, p.d.scale, qok ? p.taus[row] : 0.0f, qok);  // invalid rows: p = 0
+  // as in forward_kernel: key blocks up to qmin are visible to every row
+  int qmin;
+  {
+    const int qq = qb * kBlock + lane;
+    qmin = wave_reduce_minmax<false>(qq < NQ ? p.q_idx[size_t(bh) * NQ + qq] : INT32_MAX);
+  }
+  const int2* kbnd = p.kbounds + size_t(bh) * nKB;
+
+  f32x4 o[D / 16];
+  for (int db = 0; db < D / 16; ++db) o[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float rowsum = 0.0f;
+  uint16_t* smask = nullptr;
+  if constexpr (EMIT) smask = p.sup.mask + size_t(bh) * nQB * nKB * 256 + w * 64 + 4 * c16 + g;
+  const uint8_t* hrow = nullptr;
+  bool hvalid = true;
+  if constexpr (HALF) {
+    const int h = 2 * qb + (w >> 1), nQH = half_blocks(NQ);
+    hvalid = h < nQH;
+    hrow = p.half + (size_t(bh) * nQH + (hvalid ? h : 0)) * nKB;
+  }
+  const int32_t* qp = p.q_ptr + size_t(bh) * (nQB + 1);
+  const int32_t* ql = p.q_list + size_t(bh) * nQB * nKB;
+  const int e0 = qp[qb], e1 = qp[qb + 1];
+  St st;
+  PosStager ps;
+  auto fetch = [&](int e) {
+    const int kbase = ql[e] * kBlock;
+    st.template load<kRowsStrided>(Kb, p.lk.sn, Vb, p.lv.sn, kbase, NK, hd, t);
+    ps.load(kidx, kbase, NK, INT32_MAX, t);
+  };
+  // the staged quads, split, to the planes (a quad's four floats are half
+  // of a plane's 16-byte chunk)
+  auto put = [&](int step) {
+    uint32_t low = ~0u;
+    for (int i = 0; i < St::kPer; ++i)
+      for (int j = 0; j < 4; ++j) low = split_min(low, __builtin_bit_cast(f32x4, st.r[i][j]));
+    if (split_low(low)) sm.low[0] = step + 1;
+    for (int i = 0; i < St::kPer; ++i) {
+      const int qi = t + i * kThreads;
+      const int job = qi / St::kQuads, qd = qi % St::kQuads;
+      const int rq = qd / St::kCpr, cc = qd % St::kCpr;
+      u16* dst = (job == 0 ? sm.K[0] : sm.V[0]) + 4 * rq * kRs + ((4 * cc) ^ Tile<u16, D>::sw(4 * rq));
+      for (int j = 0; j < 4; j += 2) {
+        const Split8 x = split8(__builtin_bit_cast(f32x4, st.r[i][j]), __builtin_bit_cast(f32x4, st.r[i][j + 1]));
+        const bf16x8* pl[3] = {&x.h, &x.m, &x.l};
+        for (int y = 0; y < 3; ++y) {
+          const uint4 v = __builtin_bit_cast(uint4, *pl[y]);
+          u16* d = dst + y * (kBlock * kRs) + j * kRs;
+          *reinterpret_cast<uint2*>(d) = uint2{v.x, v.y};
+          *reinterpret_cast<uint2*>(d + kRs) = uint2{v.z, v.w};
+        }
+      }
+    }
+    ps.store(sm.kid, t);
+  };
+  const int first = e0 + grp, steps = (e1 - e0 + G - 1) / G;  // block-uniform
+  if (first < e1) fetch(first);
+  if (t == 0) sm.low[0] = 0;
+  const bool qlow = __any(split_low(qf.low));
+  for (int i = 0; i < steps; ++i) {
+    const int e = first + G * i;
+    const bool have = e < e1;  // group-uniform
+    __syncthreads();           // the previous tile's reads are done
+    if (have) put(i);
+    if (e + G < e1) fetch(e + G);
+    __syncthreads();
+    if (!have) continue;
+    const int kb = ql[e];
+    bool act = true;  // wave-uniform
+    if constexpr (HALF) act = hvalid && hrow[kb] != 0;
+    if (!act) {
+      if constexpr (EMIT) smask[size_t(e) * 256] = 0;
+      continue;
+    }
+    f32x4 acc[4];
+    for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int kat = c16 * kRs + ((8 * g) ^ Tile<u16, D>::sw(c16));
+    for (int s = 0; s < D / 32; ++s) {
+      Split8 ka[4];
+      for (int f = 0; f < 4; ++f) {
+        const int at = kat + 16 * f * kRs + 32 * s;
+        ka[f].h = *reinterpret_cast<const bf16x8*>(sm.K[0] + at);
+        ka[f].m = *reinterpret_cast<const bf16x8*>(sm.K[1] + at);
+        ka[f].l = *reinterpret_cast<const bf16x8*>(sm.K[2] + at);
+      }
+      mfma_split<4>(acc, ka, qf.v[s]);
+    }
+    const bool low = sm.low[0] == i + 1;  // group-uniform
+    if (any_nonfinite(acc) || low || qlow) {  // wave-uniform: fp32 products of the same tile
+      RowFrag<float, D> q32;
+      q32.load(qrow, qok, lane, hd);
+      rows_x_frag_global<D>(acc, Kb + size_t(kb) * kBlock * p.lk.sn, NK - kb * kBlock, size_t(p.lk.sn), hd, q32, lane);
+    }
+    auto weights = [&](auto partial) {  // as in forward_kernel
+      uint32_t nm = 0;
+      for (int f = 3; f >= 0; --f)
+        for (int r = 3; r >= 0; --r) {
+          float v = clip(acc[f][r]);
+          if constexpr (decltype(partial)::value)
+            v = sm.kid[16 * f + 4 * g + r] <= qpos ? v : -0.0f;
+          acc[f][r] = v;
+          if constexpr (EMIT) nm = __builtin_amdgcn_alignbit(nm, __float_as_uint(v), 31);
+        }
+      if constexpr (EMIT) smask[size_t(e) * 256] = uint16_t(~nm);
+      for (int f = 0; f < 4; ++f)
+        for (int r = 0; r < 4; ++r) {
+          acc[f][r] = pow_clipped<PC>(acc[f][r], a);
+          rowsum += acc[f][r];
+        }
+    };
+    if (kb * kBlock + kBlock <= NK && kbnd[kb].y <= qmin) weights(std::false_type{});
+    else weights(std::true_type{});
+    if (low) {
+      for (int f = 0; f < 4; ++f)
+        for (int r = 0; r < 4; ++r) {
+          const int key = kb * kBlock + 16 * f + 4 * g + r;
+          for (int db = 0; db < D / 16; ++db) {
+            const int col = 16 * db + c16;
+            const float v = key < NK && col < hd ? Vb[size_t(key) * p.lv.sn + col] : 0.0f;
+            o[db] = mfma(v, acc[f][r], o[db]);
+          }
+        }
+      continue;
+    }
+    for (int cc = 0; cc < 2; ++cc) {
+      const Split8 pb = split8(acc[2 * cc], acc[2 * cc + 1]);
+      const int l16 = lane & 15;
+      const int vat = (32 * cc + 4 * g + (l16 >> 2)) * kRs + ((4 * (l16 & 3)) ^ Tile<u16, D>::sw(4 * g));
+      Split8 va[D / 16];
+      auto tr = [&](int y, int db) {
+        const bf16x4 lo = read_tr16(sm.V[y] + vat + 16 * db);
+        const bf16x4 hi = read_tr16(sm.V[y] + vat + 16 * kRs + 16 * db);
+        return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      };
+      for (int db = 0; db < D / 16; ++db) {
+        va[db].h = tr(0, db);
+        va[db].m = tr(1, db);
+        va[db].l = tr(2, db);
+      }
+      mfma_split<D / 16>(o, va, pb);
+    }
+  }
+
+  if constexpr (G == 2) {  // the second group's sums to the first
+    __syncthreads();
+    constexpr int kPer = D / 16 * 4 + 1;  // floats per lane
+    float* sums = reinterpret_cast<float*>(smem_split);
+    if (grp == 1) {
+      for (int db = 0; db < D / 16; ++db)
+        for (int r = 0; r < 4; ++r) sums[(4 * db + r) * kThreads + t] = o[db][r];
+      sums[(kPer - 1) * kThreads + t] = rowsum;
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    for (int db = 0; db < D / 16; ++db)
+      for (int r = 0; r < 4; ++r) o[db][r] += sums[(4 * db + r) * kThreads + t];
+    rowsum += sums[(kPer - 1) * kThreads + t];
+  }
+  const float norm = sum_groups(rowsum);
+  const float inv = 1.0f / (norm + kEps);
+  if (qok) {
+    float* orow = static_cast<float*>(p.out) + head_at(p.lo, bh, H) + size_t(q) * p.lo.sn;
+    for (int db = 0; db < D / 16; ++db)
+      if (16 * db + 4 * g < hd) {
+        f32x4 v;
+        for (int r = 0; r < 4; ++r) {
+          v[r] = o[db][r] * inv;
+          if (!finite(v[r])) v[r] = 0.0f;
+        }
+        *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * g) = v;
+      }
+    if (g == 0) p.norms[row] = norm;
+  }
+}
+
+template <int D, int PC, bool EMIT, bool HALF, int G>
+hipError_t launch_f32_g(const ForwardParams& p, hipStream_t s) {
+  auto kern = forward_kernel<D, PC, EMIT, HALF, G>;
+  constexpr int bytes = G * int(sizeof(SplitFwdSmem<D>));
+  if (bytes > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(kern, dim3(p.d.nQB * p.d.BH), dim3(G * kThreads), bytes, s, p);
+  return hipGetLastError();
+}
+// The split forward applies where its output is smooth in the scores, which
+// it rounds differently (more closely) than the score pass that tau came
+// from: with k = 1 tau can lie within a rounding of the top score, and above
+// alpha = 2 the weights have unbounded slope at the support's edge.
+inline bool split_ok(const ForwardParams& p) { return p.d.k >= 2 && p.d.alpha <= 2.0f; }
+
+// Two groups per block while the query blocks do not exceed the compute
+// units (then each would run one wave per SIMD).
+template <int D, int PC, bool EMIT, bool HALF>
+hipError_t launch_f32(const ForwardParams& p, hipStream_t s) {
+  if (size_t(p.d.nQB) * size_t(p.d.BH) <= size_t(p.cus)) return launch_f32_g<D, PC, EMIT, HALF, 2>(p, s);
+  return launch_f32_g<D, PC, EMIT, HALF, 1>(p, s);
+}
+
 // Two query blocks per workgroup (16-bit inputs): wave w holds rows
 // 16w..16w+15 of both query blocks 2m and 2m+1, as two B fragments, and the
 // workgroup walks the union of the two blocks' key-block lists (merged on
@@ -442,14 +691,23 @@ template <typename T, int D, bool EMIT, bool HALF>
 hipError_t launch_tde(const ForwardParams& p, hipStream_t s) {
   if constexpr (is_half<T>)
     if (pair_fold_ok(p) && pair_pays(p)) return launch_pair<T, D, EMIT, HALF>(p, s);
-  dim3 grid(p.d.nQB * p.d.BH);
-  switch (alpha_class_of(p.d.alpha)) {
-    case kA15: hipLaunchKernelGGL((forward_kernel<T, D, kE2, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
-    case kA20: hipLaunchKernelGGL((forward_kernel<T, D, kE1, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
-    case kA125: hipLaunchKernelGGL((forward_kernel<T, D, kE4, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
-    default: hipLaunchKernelGGL((forward_kernel<T, D, kEGen, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
+  if constexpr (std::is_same<T, float>::value && D == 64)
+    if (split_ok(p)) switch (alpha_class_of(p.d.alpha)) {
+      case kA15: return launch_f32<D, kE2, EMIT, HALF>(p, s);
+      case kA20: return launch_f32<D, kE1, EMIT, HALF>(p, s);
+      case kA125: return launch_f32<D, kE4, EMIT, HALF>(p, s);
+      default: return launch_f32<D, kEGen, EMIT, HALF>(p, s);
+    }
+  {
+    dim3 grid(p.d.nQB * p.d.BH);
+    switch (alpha_class_of(p.d.alpha)) {
+      case kA15: hipLaunchKernelGGL((forward_kernel<T, D, kE2, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
+      case kA20: hipLaunchKernelGGL((forward_kernel<T, D, kE1, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
+      case kA125: hipLaunchKernelGGL((forward_kernel<T, D, kE4, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
+      default: hipLaunchKernelGGL((forward_kernel<T, D, kEGen, EMIT, HALF>), grid, dim3(kThreads), 0, s, p); break;
+    }
+    return hipGetLastError();
   }
-  return hipGetLastError();
 }
 template <typename T, int D>
 hipError_t launch_td(const ForwardParams& p, hipStream_t s) {
