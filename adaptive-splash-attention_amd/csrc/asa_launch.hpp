@@ -213,6 +213,16 @@ hipError_t launch_bwd_dkdv(const BackwardParams& p, int dtype, hipStream_t s);
 hipError_t launch_bwd_dq_sparse(const BackwardParams& p, int dtype, hipStream_t s);
 hipError_t launch_bwd_dkdv_sparse(const BackwardParams& p, int dtype, hipStream_t s);
 
+// Up to three tensors of n[i] elements: flags |= (1: some NaN | 2: some
+// infinity) << (2 i).
+struct NonfiniteParams {
+  int count;
+  const void* t[3];
+  size_t n[3];
+  uint32_t* flags;
+};
+hipError_t launch_nonfinite(const NonfiniteParams& p, int dtype, hipStream_t s);
+
 // Kernel-timing hooks implemented in capi.cpp (no-ops unless profiling).
 void profile_begin(const char* name, hipStream_t s);
 void profile_end(hipStream_t s);

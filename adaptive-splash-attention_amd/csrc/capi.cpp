@@ -671,6 +671,33 @@ int asa_select_from_scores(const asa_problem* p, const float* scores, const int3
   return ok();
 }
 
+int asa_check_nonfinite(int32_t dtype, int32_t count, const void* const* tensors,
+                        const int64_t* elements, uint32_t* flags, void* stream) {
+  if (dtype != ASA_DTYPE_F32 && dtype != ASA_DTYPE_BF16 && dtype != ASA_DTYPE_F16)
+    return fail(ASA_ERR_INVALID_ARGUMENT, "unknown dtype %d", dtype);
+  if (count < 1 || count > 3)
+    return fail(ASA_ERR_INVALID_ARGUMENT, "count (%d) must be 1 to 3", count);
+  if (!tensors || !elements || !flags)
+    return fail(ASA_ERR_INVALID_ARGUMENT, "an argument is NULL");
+  asa::NonfiniteParams np{};
+  np.count = count;
+  np.flags = flags;
+  for (int i = 0; i < count; ++i) {
+    if (!tensors[i] || elements[i] < 0)
+      return fail(ASA_ERR_INVALID_ARGUMENT, "tensor %d is NULL or has %lld elements", i,
+                  (long long)elements[i]);
+    if (int rc = check_aligned({tensors[i]})) return rc;
+    np.t[i] = tensors[i];
+    np.n[i] = size_t(elements[i]);
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  asa::profile_begin("nonfinite", s);
+  hipError_t e = asa::launch_nonfinite(np, dtype, s);
+  asa::profile_end(s);
+  if (int rc = check_hip(e, "nonfinite kernel launch")) return rc;
+  return ok();
+}
+
 int asa_set_pairing(int mode) {
   if (mode != ASA_PAIRING_AUTO && mode != ASA_PAIRING_ALWAYS && mode != ASA_PAIRING_NEVER)
     return fail(ASA_ERR_INVALID_ARGUMENT, "unknown pairing mode %d", mode);

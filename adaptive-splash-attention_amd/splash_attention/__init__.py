@@ -62,7 +62,7 @@ def forward(Q, K, V, Q_idx, K_idx, sm_scale: float, alpha: float, k_keep: int = 
     out, _ = ops.splash_forward(Q, K, V, qi, ki, ops.clamp_alpha(alpha), k_keep, sm_scale,
                                 with_support=False, block_m=block_m)
     out = ops.from_kernel_layout(out, d, dtype)
-    if fix_nonfinite:
+    if fix_nonfinite and ops.nonfinite([out])[0]:
         out = ops.fix_nonfinite(out, "output")
     return out
 
@@ -90,5 +90,8 @@ def backward(Q, K, V, Q_idx, K_idx, sm_scale: float, alpha: float, dOut, k_keep:
     grads = ops.splash_backward(Q, K, V, qi, ki, out, dOut, st, a, k_keep, sm_scale, grad_mode)
     grads = [ops.from_kernel_layout(g, d, dtype) for g in grads]
     if fix_nonfinite:
-        grads = [ops.fix_nonfinite(g, n) for g, n in zip(grads, ("dQ", "dK", "dV"))]
+        bad = ops.nonfinite(grads)
+        for i, n in enumerate(("dQ", "dK", "dV")):
+            if bad[i]:
+                grads[i] = ops.fix_nonfinite(grads[i], n)
     return grads

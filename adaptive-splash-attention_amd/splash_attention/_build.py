@@ -21,7 +21,7 @@ LIBDIR = os.path.join(PKG_DIR, "lib")
 LIB = os.path.join(LIBDIR, "libadasplash.so")
 
 SOURCES = ["sparse_bwd.hip", "select_bf16.hip", "select_f16.hip", "select_f32.hip", "forward.hip",
-           "backward.hip", "exact.hip", "select.hip", "compact.hip", "capi.cpp"]
+           "backward.hip", "exact.hip", "select.hip", "compact.hip", "check.hip", "capi.cpp"]
 ARCH = "gfx950"
 FLAGS = [
     f"--offload-arch={ARCH}",

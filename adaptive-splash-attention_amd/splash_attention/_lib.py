@@ -44,6 +44,7 @@ EXPORTS = (
     "asa_forward_noalloc",
     "asa_backward",
     "asa_select_from_scores",
+    "asa_check_nonfinite",
     "asa_set_pairing",
     "asa_profile_enable",
     "asa_profile_read",
@@ -148,6 +149,8 @@ def load() -> ctypes.CDLL:
         lib.asa_select_from_scores.restype = ctypes.c_int
         lib.asa_select_from_scores.argtypes = [ctypes.POINTER(Problem), _V, _V, _V,
                                                ctypes.POINTER(State), _V, _V]
+        lib.asa_check_nonfinite.restype = ctypes.c_int
+        lib.asa_check_nonfinite.argtypes = [_I, _I, _V, _V, _V, _V]
         lib.asa_set_pairing.restype = ctypes.c_int
         lib.asa_set_pairing.argtypes = [ctypes.c_int]
         lib.asa_profile_enable.restype = ctypes.c_int

@@ -139,6 +139,26 @@ def fix_nonfinite(t: torch.Tensor, name: str) -> torch.Tensor:
     return t
 
 
+def nonfinite(ts) -> list:
+    """For each of up to three tensors, whether it needs fix_nonfinite (it may
+    hold a NaN or an infinity): one scan of all of them and one word read
+    back, where fix_nonfinite reads two reductions back per tensor."""
+    t0 = ts[0]
+    if not all(t.is_cuda and t.is_contiguous() and t.device == t0.device and t.dtype == t0.dtype
+               and t.dtype in _DTYPES and t.numel() and t.data_ptr() % 16 == 0 for t in ts):
+        return [True] * len(ts)
+    flags = torch.zeros((1,), dtype=torch.int32, device=t0.device)
+    n = len(ts)
+    ptrs = (ctypes.c_void_p * n)(*(t.data_ptr() for t in ts))
+    sizes = (ctypes.c_int64 * n)(*(t.numel() for t in ts))
+    with torch.cuda.device(t0.device):
+        rc = _lib.load().asa_check_nonfinite(_DTYPES[t0.dtype], n, ptrs, sizes, flags.data_ptr(),
+                                             _stream(t0.device))
+    _lib.check(rc)
+    word = int(flags.item())
+    return [(word >> (2 * i)) & 3 != 0 for i in range(n)]
+
+
 def clamp_alpha(alpha: float) -> float:
     """alpha as the kernels use it (adasplashattention.cu:547)."""
     return max(1.05, min(float(alpha), 3.0))

@@ -262,6 +262,14 @@ int asa_select_from_scores(const asa_problem *p, const float *scores, const int3
  * them and reports, per kernel name, the number of launches and the summed
  * duration in milliseconds, then clears the record.  Call it when no other
  * thread is launching.  Returns the number of distinct kernels (<= max).  */
+/* Scans up to three 16-byte aligned tensors of elements[i] values of one
+ * dtype for the reference's host fix-up (adasplashattention.cu:599-606,
+ * :684-697): ORs (1 if tensor i holds a NaN, 2 if it holds an infinity)
+ * << (2 i) into the device word *flags, which the caller has cleared on
+ * `stream`. */
+int asa_check_nonfinite(int32_t dtype, int32_t count, const void* const* tensors,
+                        const int64_t* elements, uint32_t* flags, void* stream);
+
 /* Which forward kernel runs for 16-bit inputs (no reference counterpart;
  * for tuning and tests): ASA_PAIRING_AUTO (default) runs two query blocks
  * per workgroup when those workgroups fill at least one wave of the GPU
