@@ -31,7 +31,9 @@ class SplashAttentionFunction(torch.autograd.Function):
                                                    and bwd_passes == "support"),
                                      tau_mode=tau_mode, block_m=block_m)
         ctx.params = (alpha, k_keep, sm_scale, grad_mode)
-        ctx.save_for_backward(Q, K, V, Q_idx, K_idx, out, *st.tensors())
+        # the output only where the backward reads it (the reference gradient)
+        ctx.save_for_backward(Q, K, V, Q_idx, K_idx, out if grad_mode == "reference" else None,
+                              *st.tensors())
         return out
 
     @staticmethod

@@ -170,6 +170,9 @@ def _stream(dev: torch.device) -> int:
 
 def _index(idx, BH: int, N: int, B: int, H: int, device, name: str) -> torch.Tensor:
     """Position indices as int32 [BH, N] on `device` (reference: Q_idx/K_idx [B*H, N])."""
+    if (type(idx) is torch.Tensor and idx.dtype == torch.int32 and idx.shape == (BH, N)
+            and idx.device == device and idx.is_contiguous()):
+        return idx
     if idx is None:
         return torch.arange(N, device=device, dtype=torch.int32).unsqueeze(0).expand(BH, N).contiguous()
     if not isinstance(idx, torch.Tensor):
@@ -298,23 +301,44 @@ def strides_of(t: torch.Tensor) -> tuple:
     return tuple(st if n > 1 else c for n, st, c in zip((B, H, N), t.stride()[:3], contiguous))
 
 
+def _plain_operand(t: torch.Tensor) -> bool:
+    """Whether a [B, H, N, d] operand is the common case of readable_in_place:
+    contiguous, aligned, whole chunks, a head's rows within 2^31 bytes (one
+    call each instead of the stride arithmetic; the ABI's zero strides)."""
+    d, es = t.size(-1), t.element_size()
+    return (t.is_contiguous() and t.data_ptr() % 16 == 0 and d * es % 16 == 0
+            and t.size(2) * d * es < 2 ** 31)
+
+
+def _readable_strides(t: torch.Tensor):
+    """The strides to pass for a [B, H, N, d] operand that the kernels can
+    read where it is (the C ABI's stride rules, asa_problem.q_strides): ()
+    for the common contiguous case (the ABI's zeros), else strides_of;
+    None if they cannot."""
+    if _plain_operand(t):
+        return ()
+    B, H, N, d = t.shape
+    es = t.element_size()
+    e = 16 // es
+    sb, sh, sn, sd = t.stride()
+    if (d > 1 and sd != 1) or t.data_ptr() % 16:
+        return None
+    # as strides_of
+    sb, sh, sn = sb if B > 1 else H * N * d, sh if H > 1 else N * d, sn if N > 1 else d
+    if sb < 0 or sh < 0 or sn < 0 or sb % e or sh % e or sn % e:
+        return None
+    if sb == sh == sn == 0:  # broadcast along batch, heads and rows: the ABI's "contiguous" mark
+        return None
+    return (sb, sh, sn) if ((N - 1) * sn + d) * es < 2 ** 31 else None
+
+
 def readable_in_place(t: torch.Tensor) -> bool:
     """Whether the kernels can read a [B, H, N, d] operand where it is (the
     C ABI's stride rules, asa_problem.q_strides): contiguous head dimension,
     16-byte aligned start, non-negative batch, head and row strides that are
     whole 16-byte chunks, not all three 0, and a head's rows within 2^31
     bytes of its first."""
-    e = chunk_elems(t.dtype)
-    if t.size(-1) > 1 and t.stride(-1) != 1:
-        return False
-    if t.data_ptr() % 16:
-        return False
-    st = strides_of(t)
-    if any(x < 0 or x % e for x in st):
-        return False
-    if st == (0, 0, 0):  # broadcast along batch, heads and rows: the ABI's "contiguous" mark
-        return False
-    return ((t.size(2) - 1) * st[2] + t.size(-1)) * t.element_size() < 2 ** 31
+    return _readable_strides(t) is not None
 
 
 def kernel_operand(t: torch.Tensor) -> torch.Tensor:
@@ -340,12 +364,12 @@ def _set_strides(p: _lib.Problem, **ts) -> None:
     operand the kernels cannot read in place (pass it through check_inputs
     or kernel_operand first)."""
     for name, t in ts.items():
-        if not readable_in_place(t):
+        st = _readable_strides(t)
+        if st is None:
             raise ValueError(f"{name}: shape {tuple(t.shape)} with strides {tuple(t.stride())} "
                              "cannot be read in place; pass it through check_inputs first")
         arr = getattr(p, name + "_strides")
-        for i, x in enumerate(strides_of(t)):
-            arr[i] = x
+        arr[:] = st or (0, 0, 0)
 
 
 def check_tau_mode(tau_mode: str) -> int:
@@ -372,6 +396,21 @@ def block_m_of(st: "SplashState", NQ: int) -> int:
     """The block_m a state was written with, from its mask's row count (for
     NQ <= 32 both give one identical row; 64 is returned)."""
     return 64 if st.mask.shape[1] == -(-NQ // 64) else 32
+
+
+class _on_device:
+    """torch.cuda.device(dev) that is free where dev is current already."""
+
+    def __init__(self, dev: torch.device):
+        self.ctx = None if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+    def __enter__(self):
+        if self.ctx is not None:
+            self.ctx.__enter__()
+
+    def __exit__(self, *exc):
+        if self.ctx is not None:
+            self.ctx.__exit__(*exc)
 
 
 def make_problem(B, H, NQ, NK, d, dtype, alpha, k_keep, sm_scale,
@@ -440,14 +479,14 @@ def splash_forward(Q, K, V, Q_idx, K_idx, alpha: float, k_keep: int, sm_scale=No
     out = torch.empty(Q.shape, dtype=Q.dtype, device=Q.device)
     cst = st.c_struct()
     if noalloc:
-        with torch.cuda.device(Q.device):
+        with _on_device(Q.device):
             rc = lib.asa_forward_noalloc(ctypes.byref(p), Q.data_ptr(), K.data_ptr(), V.data_ptr(),
                                          Q_idx.data_ptr(), K_idx.data_ptr(), out.data_ptr(),
                                          ctypes.byref(cst), _stream(Q.device))
         _lib.check(rc)
         return out, st
     ws = workspace(p, Q.device)
-    with torch.cuda.device(Q.device):
+    with _on_device(Q.device):
         rc = lib.asa_forward(ctypes.byref(p), Q.data_ptr(), K.data_ptr(), V.data_ptr(),
                              Q_idx.data_ptr(), K_idx.data_ptr(), out.data_ptr(),
                              ctypes.byref(cst), ws.data_ptr(), _stream(Q.device))
@@ -463,6 +502,8 @@ def _as_kernel_operand(t: torch.Tensor, Q: torch.Tensor, name: str, contiguous: 
     if (t.dim() != 4 or tuple(t.shape[:3]) != tuple(Q.shape[:3]) or t.size(-1) > dq
             or kernel_head_dim(t.size(-1), Q.dtype) != dq):
         raise ValueError(f"{name} shape {tuple(t.shape)} must equal Q shape {tuple(Q.shape)}")
+    if t.dtype == Q.dtype and t.shape == Q.shape and _plain_operand(t):
+        return t
     (t,) = to_kernel_layout(t.to(Q.dtype))
     return _aligned(t) if contiguous else kernel_operand(t)
 
@@ -485,7 +526,7 @@ def splash_backward(Q, K, V, Q_idx, K_idx, out, dout, st: SplashState, alpha: fl
     dK = torch.empty(K.shape, dtype=K.dtype, device=K.device)
     dV = torch.empty(V.shape, dtype=V.dtype, device=V.device)
     cst = st.c_struct()
-    with torch.cuda.device(Q.device):
+    with _on_device(Q.device):
         rc = lib.asa_backward(ctypes.byref(p), GRAD_MODES[grad_mode], Q.data_ptr(), K.data_ptr(),
                               V.data_ptr(), Q_idx.data_ptr(), K_idx.data_ptr(),
                               None if out is None else out.data_ptr(), dout.data_ptr(),
