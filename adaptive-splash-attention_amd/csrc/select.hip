@@ -1,6 +1,7 @@
 // Key-block position bounds, tau from the sorted top-k values, and the
 // dispatch of the score pass (select_kernel.hpp) by storage type.
 #include <climits>
+#include <type_traits>
 
 #include "asa_compact.hpp"
 #include "asa_device.hpp"
@@ -190,28 +191,33 @@ hipError_t launch_bounds(const SelectParams& p, hipStream_t s) {
   return hipGetLastError();
 }
 
+// f(AC, KMAX) for the problem's exponent class and the fewest register slots
+// that hold a row's k values (0: read from memory).  The sums run over every
+// slot, so their number sets a launch's time where it has few rows: at
+// k = 8, 8 slots against 32 took the tau and compaction launch from 14.0 to
+// 7.0 us at 2x8x1024 rows (k = 16, 3x5x1537: 14.4 -> 9.4 us).
+template <typename F>
+void with_tau_variant(const Dims& d, F&& f) {
+  auto slots = [&](auto ac) {
+    if (d.k <= 8) f(ac, std::integral_constant<int, 8>{});
+    else if (d.k <= 16) f(ac, std::integral_constant<int, 16>{});
+    else if (d.k <= 32) f(ac, std::integral_constant<int, 32>{});
+    else f(ac, std::integral_constant<int, 0>{});
+  };
+  switch (alpha_class_of(d.alpha)) {
+    case kA15: slots(std::integral_constant<int, kA15>{}); break;
+    case kA20: slots(std::integral_constant<int, kA20>{}); break;
+    case kA125: slots(std::integral_constant<int, kA125>{}); break;
+    default: slots(std::integral_constant<int, kAGen>{}); break;
+  }
+}
+
 hipError_t launch_tau(const SelectParams& p, hipStream_t s) {
   const size_t rows = size_t(p.d.BH) * p.d.NQ;
   const dim3 grid(unsigned((rows + kThreads - 1) / kThreads));
-  const bool reg = p.d.k <= 32;  // the row's values fit in registers
-  switch (alpha_class_of(p.d.alpha)) {
-    case kA15:
-      if (reg) hipLaunchKernelGGL((tau_kernel<kA15, 32>), grid, dim3(kThreads), 0, s, p);
-      else hipLaunchKernelGGL((tau_kernel<kA15, 0>), grid, dim3(kThreads), 0, s, p);
-      break;
-    case kA20:
-      if (reg) hipLaunchKernelGGL((tau_kernel<kA20, 32>), grid, dim3(kThreads), 0, s, p);
-      else hipLaunchKernelGGL((tau_kernel<kA20, 0>), grid, dim3(kThreads), 0, s, p);
-      break;
-    case kA125:
-      if (reg) hipLaunchKernelGGL((tau_kernel<kA125, 32>), grid, dim3(kThreads), 0, s, p);
-      else hipLaunchKernelGGL((tau_kernel<kA125, 0>), grid, dim3(kThreads), 0, s, p);
-      break;
-    default:
-      if (reg) hipLaunchKernelGGL((tau_kernel<kAGen, 32>), grid, dim3(kThreads), 0, s, p);
-      else hipLaunchKernelGGL((tau_kernel<kAGen, 0>), grid, dim3(kThreads), 0, s, p);
-      break;
-  }
+  with_tau_variant(p.d, [&](auto ac, auto kmax) {
+    hipLaunchKernelGGL((tau_kernel<decltype(ac)::value, decltype(kmax)::value>), grid, dim3(kThreads), 0, s, p);
+  });
   return hipGetLastError();
 }
 
@@ -221,25 +227,10 @@ hipError_t launch_tau_compact(const SelectParams& p, const CompactParams& cp, hi
   const int ncomp = compact_detail::compact_grid(cp);
   const dim3 grid(unsigned(ntau + ncomp));
   const size_t lds = compact_detail::compact_lds_bytes(cp);
-  const bool reg = p.d.k <= 32;  // the row's values fit in registers
-  switch (alpha_class_of(p.d.alpha)) {
-    case kA15:
-      if (reg) hipLaunchKernelGGL((tau_compact_kernel<kA15, 32>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      else hipLaunchKernelGGL((tau_compact_kernel<kA15, 0>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      break;
-    case kA20:
-      if (reg) hipLaunchKernelGGL((tau_compact_kernel<kA20, 32>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      else hipLaunchKernelGGL((tau_compact_kernel<kA20, 0>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      break;
-    case kA125:
-      if (reg) hipLaunchKernelGGL((tau_compact_kernel<kA125, 32>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      else hipLaunchKernelGGL((tau_compact_kernel<kA125, 0>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      break;
-    default:
-      if (reg) hipLaunchKernelGGL((tau_compact_kernel<kAGen, 32>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      else hipLaunchKernelGGL((tau_compact_kernel<kAGen, 0>), grid, dim3(kThreads), lds, s, p, cp, ncomp);
-      break;
-  }
+  with_tau_variant(p.d, [&](auto ac, auto kmax) {
+    hipLaunchKernelGGL((tau_compact_kernel<decltype(ac)::value, decltype(kmax)::value>), grid, dim3(kThreads),
+                       lds, s, p, cp, ncomp);
+  });
   return hipGetLastError();
 }
 

@@ -166,7 +166,7 @@ def test_select_ties_beyond_the_list_bit_exact(dev, k, with_topk):
 
 
 @pytest.mark.parametrize("layout", ["dense", "rows"])
-@pytest.mark.parametrize("k", [1, 32, 42, 43, 64, 65, 128])
+@pytest.mark.parametrize("k", [1, 8, 9, 16, 17, 32, 42, 43, 64, 65, 128])
 @pytest.mark.parametrize("d,dtype", [(64, torch.bfloat16), (128, torch.bfloat16), (128, torch.float16),
                                      (96, torch.bfloat16), (64, torch.float32), (128, torch.float32)])
 def test_score_pass_variants(dev, d, dtype, k, layout):
@@ -200,3 +200,36 @@ def test_score_pass_variants(dev, d, dtype, k, layout):
     for st in got:
         np.testing.assert_array_equal(st.mask.cpu().numpy(), sel.mask)
         np.testing.assert_array_equal(st.taus.cpu().numpy(), sel.taus)
+
+
+@pytest.mark.parametrize("d,dtype,k", [(128, torch.bfloat16, 32), (128, torch.float16, 64),
+                                       (64, torch.bfloat16, 128), (64, torch.float32, 8)])
+def test_captured_variants(dev, d, dtype, k):
+    """The variants with more than 64 KiB of LDS (and the two-group fp32
+    forward) captured in a graph: every replay on new inputs, with eager work
+    between, bit-equal to the eager call."""
+    import splash_attention as sa
+
+    B, H, N = 1, 2, 700
+    print(f"[select] captured d={d} {dtype} k={k}", flush=True)
+    idx = causal_idx(B * H, N).to(dev)
+    g = torch.Generator(device=dev).manual_seed(d + k)
+    new = lambda: torch.randn(B, H, N, d, generator=g, device=dev).to(dtype)
+    bufs = [new() for _ in range(3)]
+    call = lambda q, kk, v: sa.splash_attention(q, kk, v, idx, idx, 1.5, k)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(*bufs)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call(*bufs)
+    for _ in range(3):
+        fresh = [new() for _ in range(3)]
+        want = call(*fresh)
+        for b, f in zip(bufs, fresh):
+            b.copy_(f)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
