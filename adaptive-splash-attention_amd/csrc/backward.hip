@@ -52,20 +52,37 @@ constexpr int kThreads = 256;
 // ---------------------------------------------------------------------------
 // Row constants for the reference-gradient mode.
 // ---------------------------------------------------------------------------
+// shift = out . dO and 1 / (sum p + EPS) per row.  HBM-bound by bytes (Out
+// and dO once); a group of lanes takes 16 bytes of the row each, so that a
+// wave reads whole rows (one thread per row read 64 separate lines per load
+// and walked the row serially: 20.5 -> 6.9 us at 1x6x1500x64 fp32).
 template <typename T, int D>
 __global__ __launch_bounds__(kThreads) void delta_kernel(BackwardParams p) {
+  constexpr int E = 16 / int(sizeof(T)), LPR = D / E;  // lanes per row: 8, 16 or 32
   const size_t rows = size_t(p.d.BH) * p.d.NQ;
-  const size_t r = size_t(blockIdx.x) * kThreads + threadIdx.x;
-  if (r >= rows) return;
-  const int bh = int(r / p.d.NQ), n = int(r % p.d.NQ);
-  const T* o = static_cast<const T*>(p.out) + head_at(p.lo, bh, p.d.H) + size_t(n) * p.lo.sn;
-  const T* go = static_cast<const T*>(p.dout) + head_at(p.ldo, bh, p.d.H) + size_t(n) * p.ldo.sn;
+  const size_t r = size_t(blockIdx.x) * (kThreads / LPR) + threadIdx.x / LPR;
+  const int sub = threadIdx.x % LPR;
+  const bool in = r < rows;  // the same for the lanes of a row
   float acc = 0.0f;
-  for (int t = 0; t < p.d.hd; ++t) acc += Elem<T>::load(o + t) * Elem<T>::load(go + t);
-  float* shift = p.delta;
-  float* cfac = p.delta + rows;
-  shift[r] = acc;
-  cfac[r] = 1.0f / (p.norms[r] + kEps);
+  if (in && sub * E < p.d.hd) {
+    const int bh = int(r / p.d.NQ), n = int(r % p.d.NQ);
+    const T* o = static_cast<const T*>(p.out) + head_at(p.lo, bh, p.d.H) + size_t(n) * p.lo.sn + sub * E;
+    const T* go = static_cast<const T*>(p.dout) + head_at(p.ldo, bh, p.d.H) + size_t(n) * p.ldo.sn + sub * E;
+    alignas(16) T x[E], y[E];
+    *reinterpret_cast<uint4*>(x) = *reinterpret_cast<const uint4*>(o);
+    *reinterpret_cast<uint4*>(y) = *reinterpret_cast<const uint4*>(go);
+    for (int i = 0; i < E; ++i) acc = fmaf(Elem<T>::load(x + i), Elem<T>::load(y + i), acc);
+  }
+  auto add = [&](auto m) { acc += __uint_as_float(lane_xor<decltype(m)::value>(__float_as_uint(acc))); };
+  add(std::integral_constant<int, 1>{});
+  add(std::integral_constant<int, 2>{});
+  add(std::integral_constant<int, 4>{});
+  if constexpr (LPR >= 16) add(std::integral_constant<int, 8>{});
+  if constexpr (LPR >= 32) add(std::integral_constant<int, 16>{});
+  if (in && sub == 0) {
+    p.delta[r] = acc;
+    p.delta[rows + r] = 1.0f / (p.norms[r] + kEps);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -449,7 +466,8 @@ hipError_t launch_dkdv_td(const BackwardParams& p, hipStream_t s) {
 template <typename T, int D>
 hipError_t launch_delta_td(const BackwardParams& p, hipStream_t s) {
   const size_t rows = size_t(p.d.BH) * p.d.NQ;
-  const unsigned blocks = unsigned((rows + kThreads - 1) / kThreads);
+  constexpr size_t per = kThreads * 16 / (D * sizeof(T));  // rows per block
+  const unsigned blocks = unsigned((rows + per - 1) / per);
   hipLaunchKernelGGL((delta_kernel<T, D>), dim3(blocks), dim3(kThreads), 0, s, p);
   return hipGetLastError();
 }
