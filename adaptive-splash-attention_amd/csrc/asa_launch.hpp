@@ -185,7 +185,7 @@ struct SelectPlan {
   int cap;
   size_t needs;
 };
-SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_lds);
+SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_lds, int cus);
 hipError_t launch_bounds(const SelectParams& p, hipStream_t s);
 hipError_t launch_tau(const SelectParams& p, hipStream_t s);
 // Exact-threshold pass (tau mode "exact"): after launch_tau, before

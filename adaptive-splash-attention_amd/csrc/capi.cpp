@@ -293,7 +293,9 @@ int select_plan_of(const Shape& s, bool from_scores, asa::SelectPlan* plan) {
                                                dev),
                          "hipDeviceGetAttribute"))
     return rc;
-  *plan = asa::select_plan(dims_of(s), s.dtype, from_scores, size_t(max_lds));
+  int cus = 0;
+  if (int rc = device_cus(&cus)) return rc;
+  *plan = asa::select_plan(dims_of(s), s.dtype, from_scores, size_t(max_lds), cus);
   if (plan->cap < 0)
     return fail(ASA_ERR_UNSUPPORTED, "k_keep %d needs %zu bytes of LDS per block, device has %d",
                 s.k, plan->needs, max_lds);

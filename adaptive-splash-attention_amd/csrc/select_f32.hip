@@ -9,7 +9,7 @@ hipError_t launch_select_scores(const SelectParams& p, hipStream_t s) {
   return launch_r<float, 64, kGivenScores>(p, s);
 }
 
-SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_lds) {
+SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_lds, int cus) {
   // Rings: 16-bit inputs, hd = D, raw dots (launch_ring).
   const bool raw = !from_scores && d.scale > 0.0f;
   const bool ring = raw && dtype != kElemF32 && d.hd == d.D;
@@ -18,7 +18,14 @@ SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_ld
   // 4-wave blocks fit below; 1x16x8192, d = 128, k = 32: 432 against 495 us
   // with eight).  1x8x32768, d = 128, k = 128: 4.9 -> 3.7 ms.  fp32 at
   // d = 128 holds 128 registers of Q and would spill at two waves per SIMD.
-  const bool wide = raw && (d.k > 64 || (d.k > 42 && ring && d.D == 128)) &&
+  // And where the grid gives each compute unit one block at most, whose
+  // waves then are all that the unit runs: calls of four against eight
+  // waves, 16x16 heads of 1x4096, d = 64, k = 32, bf16 104.1 -> 97.7 us;
+  // fp32, d = 64, k = 8: forward at 1x4x4096 402 -> 375 us, backward (with
+  // its forward) at 1x6x1500 281 -> 271 us.  With more blocks two 4-wave
+  // ones share a unit.
+  const bool few = size_t(d.nQB) * size_t(d.BH) <= size_t(cus);
+  const bool wide = raw && (few || d.k > 64 || (d.k > 42 && ring && d.D == 128)) &&
                     !(dtype == kElemF32 && d.D == 128);
   const struct { int waves; bool ring; } tries[] = {{wide ? 8 : 4, ring}, {4, ring}, {4, false}};
   for (const auto& t : tries) {

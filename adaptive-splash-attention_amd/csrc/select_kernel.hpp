@@ -1122,11 +1122,9 @@ hipError_t launch_ring(const SelectParams& p, hipStream_t s) {
 // Class sets per (row, position): classes_per_lane; waves: select_plan.
 template <typename T, int D, int MODE>
 hipError_t launch_r(const SelectParams& p, hipStream_t s) {
-  if constexpr (MODE == kRawDots)
-    if (p.waves == 8)
-    {
-      if constexpr (is_half<T> && D == 128)
-        if (p.d.k <= 64) return launch_ring<T, D, MODE, 1, 8>(p, s);
+  if constexpr (MODE == kRawDots && (is_half<T> || D == 64))
+    if (p.waves == 8) {
+      if (p.d.k <= 64) return launch_ring<T, D, MODE, 1, 8>(p, s);
       return launch_ring<T, D, MODE, 2, 8>(p, s);
     }
   if (p.d.k <= 64) return launch_ring<T, D, MODE, 2, 4>(p, s);

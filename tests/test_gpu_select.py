@@ -233,3 +233,37 @@ def test_captured_variants(dev, d, dtype, k):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("heads", [128, 129])
+@pytest.mark.parametrize("NK", [64 * 9 + 5, 64 * 130 + 5])
+@pytest.mark.parametrize("d,dtype,k", [(64, torch.bfloat16, 8), (64, torch.float16, 64),
+                                       (128, torch.bfloat16, 32), (96, torch.bfloat16, 16),
+                                       (64, torch.float32, 1), (64, torch.float32, 64)])
+def test_score_pass_by_block_count(dev, d, dtype, k, NK, heads):
+    """The score pass's waves per block change where the blocks exceed the
+    compute units (two blocks per head here, 256 units): both sides on short
+    and long lists against the oracle, on scores that are exact in fp32.
+    Q and K are one head's, repeated, with other positions per head."""
+    import splash_attention as sa
+
+    NQ, scale = 75, 0.125
+    print(f"[select] blocks d={d} {dtype} k={k} NK={NK} heads={heads}", flush=True)
+    g = torch.Generator().manual_seed(1000 * d + k)
+    Q, K = ((torch.round(torch.randn(1, 1, n, d, generator=g) * 16) / 16).clamp(-4, 4)
+            for n in (NQ, NK))
+    kidx = causal_idx(heads, NK)
+    qidx = torch.randint(40, NK, (1, NQ), generator=g).to(torch.int32).repeat(heads, 1)
+    qidx[1::2] = NK - 1  # odd heads see every key
+    q, kk = (x.to(dtype).to(dev).expand(1, heads, -1, -1) for x in (Q, K))
+    got = [sa.ops.splash_forward(q, kk, kk, qidx.to(dev), kidx.to(dev), 1.5, k, scale,
+                                 with_topk=t, with_support=False)[1] for t in (True, False)]
+    torch.cuda.synchronize()
+    S, vis = orc.scores(Q.repeat(1, 2, 1, 1)[0].numpy(), K.repeat(1, 2, 1, 1)[0].numpy(),
+                        qidx[:2].numpy(), kidx[:2].numpy(), scale)
+    sel = orc.select(S, vis, k, 1.5)
+    for name, sts in (("topk_idx", got[:1]), ("topk_val", got[:1]), ("mask", got), ("taus", got)):
+        for st in sts:
+            x, want = getattr(st, name).cpu().numpy(), getattr(sel, name)
+            for h in range(heads):
+                np.testing.assert_array_equal(x[h], want[h % 2])
