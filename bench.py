@@ -57,8 +57,8 @@ COPY_BYTES = 256 << 20   # --copy-calibration copy size
 # library built from the sources whose hash is HBM_TRAFFIC_SOURCES
 # (source_hash()).  A line from a library built from other sources reports
 # traffic null and says why: counters of another build are not evidence.
-HBM_TRAFFIC_SOURCES = "2d00522ce6db3e3c"
-HBM_TRAFFIC = {'bounds': 1109233, 'select': 138861915, 'tau': 34745917, 'tau_compact': 37510848, 'refine': 109582540, 'compact': 2762350, 'forward': 329894294, 'bwd_dq_sparse': 240749933, 'bwd_dkdv_sparse': 287676950}
+HBM_TRAFFIC_SOURCES = "b451c63a57f8c8eb"
+HBM_TRAFFIC = {'bounds': 1109877, 'select': 141538268, 'tau': 34740416, 'tau_compact': 37519424, 'refine': 110422821, 'compact': 2761045, 'forward': 330780416, 'bwd_dq_sparse': 240769568, 'bwd_dkdv_sparse': 287717504}
 
 
 def source_hash() -> str:
