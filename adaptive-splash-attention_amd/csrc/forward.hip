@@ -183,6 +183,19 @@ __global__ __launch_bounds__(kThreads) void forward_kernel(ForwardParams p) {
   }
 }
 
+// Blocks with a row whose best key has u = (alpha - 1) s - tau of at most this
+// take fp32 products for their scores, the rounding that tau came from.  Where
+// a row's k best scores are equal (repeated keys) the threshold recurrence
+// starts within a rounding of them and can end there, and the score's rounding
+// then decides whether the row has any weight (alpha = 2: no output, or the
+// mean of the tied keys' V).  Above the line another rounding of a score s
+// (1e-6 at most for |s| < 10) moves a weight by 1e-6 / ((alpha - 1) u) of it.
+// Below the line are rows whose recurrence did not converge in its five rounds
+// and nearly uniform ones: more than 16 equal weights at alpha = 2, 256 at
+// 1.5.  Such a block costs what forward_kernel's does (2x8x2048x64, alpha 2,
+// k = 128, 0.1 N(0, 1): 123 us, forward_kernel 128, split scores 107).
+constexpr float kSplitLeastU = 0x1p-4f;
+
 // fp32 at d <= 64 (split_ok): the one-block kernel on the bf16 matrix unit
 // (asa_tiles.hpp, split products).  K and V tiles are split into their three
 // bf16 planes once, as they are staged (55 KB of LDS for one tile pair: two
@@ -197,7 +210,10 @@ __global__ __launch_bounds__(kThreads) void forward_kernel(ForwardParams p) {
 // 1249 -> 980 us, 2x8x2048x64 125 -> 102 us, 1x4x4096x64 219 -> 150 us; the
 // output's 2-norm error against float64 falls from 1.2e-6 to 0.8e-6.
 template <int D> struct alignas(16) SplitFwdSmem {
-  u16 K[3][kBlock * Tile<u16, D>::kRs];
+  union {
+    u16 K[3][kBlock * Tile<u16, D>::kRs];
+    float K32[kBlock * Tile<float, D>::kRs];  // blocks with fp32 scores
+  };
   u16 V[3][kBlock * Tile<u16, D>::kRs];
   int kid[kBlock];
   int low[4];  // low[0]: 1 + the last step whose tiles hold a value below 2^-109
@@ -225,17 +241,21 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
   const float* Vb = static_cast<const float*>(p.v) + head_at(p.lv, bh, H);
   const int32_t* kidx = p.k_idx + size_t(bh) * NK;
   const float* qrow = static_cast<const float*>(p.q) + head_at(p.lq, bh, H) + size_t(qok ? q : 0) * p.lq.sn;
-  SplitRow<D> qf;
-  qf.load(qrow, qok, lane, hd);
   const int qpos = qok ? p.q_idx[row] : 0;
   const float am1 = p.d.alpha - 1.0f;
   const float a = 1.0f / am1;
   const SignedClip clip(am1, p.d.scale, qok ? p.taus[row] : 0.0f, qok);  // invalid rows: p = 0
-  // as in forward_kernel: key blocks up to qmin are visible to every row
+  // as in forward_kernel: key blocks up to qmin are visible to every row;
+  // and whether the block takes fp32 scores (kSplitLeastU)
   int qmin;
+  bool fp32;  // block-uniform
   {
     const int qq = qb * kBlock + lane;
-    qmin = wave_reduce_minmax<false>(qq < NQ ? p.q_idx[size_t(bh) * NQ + qq] : INT32_MAX);
+    const size_t r = size_t(bh) * NQ + (qq < NQ ? qq : 0);
+    qmin = wave_reduce_minmax<false>(qq < NQ ? p.q_idx[r] : INT32_MAX);
+    // rows without a visible key have the empty slot's score, -1e6
+    const float s1 = p.top1[r];
+    fp32 = __any(qq < NQ && s1 >= -10.0f && !(fmaf(am1, s1, -p.taus[r]) > kSplitLeastU));
   }
   const int2* kbnd = p.kbounds + size_t(bh) * nKB;
 
@@ -261,118 +281,137 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
     st.template load<kRowsStrided>(Kb, p.lk.sn, Vb, p.lv.sn, kbase, NK, hd, t);
     ps.load(kidx, kbase, NK, INT32_MAX, t);
   };
-  // the staged quads, split, to the planes (a quad's four floats are half
-  // of a plane's 16-byte chunk)
-  auto put = [&](int step) {
-    uint32_t low = ~0u;
-    for (int i = 0; i < St::kPer; ++i)
-      for (int j = 0; j < 4; ++j) low = split_min(low, __builtin_bit_cast(f32x4, st.r[i][j]));
-    if (split_low(low)) sm.low[0] = step + 1;
-    for (int i = 0; i < St::kPer; ++i) {
-      const int qi = t + i * kThreads;
-      const int job = qi / St::kQuads, qd = qi % St::kQuads;
-      const int rq = qd / St::kCpr, cc = qd % St::kCpr;
-      u16* dst = (job == 0 ? sm.K[0] : sm.V[0]) + 4 * rq * kRs + ((4 * cc) ^ Tile<u16, D>::sw(4 * rq));
-      for (int j = 0; j < 4; j += 2) {
-        const Split8 x = split8(__builtin_bit_cast(f32x4, st.r[i][j]), __builtin_bit_cast(f32x4, st.r[i][j + 1]));
-        const bf16x8* pl[3] = {&x.h, &x.m, &x.l};
-        for (int y = 0; y < 3; ++y) {
-          const uint4 v = __builtin_bit_cast(uint4, *pl[y]);
-          u16* d = dst + y * (kBlock * kRs) + j * kRs;
-          *reinterpret_cast<uint2*>(d) = uint2{v.x, v.y};
-          *reinterpret_cast<uint2*>(d + kRs) = uint2{v.z, v.w};
-        }
-      }
-    }
-    ps.store(sm.kid, t);
-  };
   const int first = e0 + grp, steps = (e1 - e0 + G - 1) / G;  // block-uniform
-  if (first < e1) fetch(first);
-  if (t == 0) sm.low[0] = 0;
-  const bool qlow = __any(split_low(qf.low));
-  for (int i = 0; i < steps; ++i) {
-    const int e = first + G * i;
-    const bool have = e < e1;  // group-uniform
-    __syncthreads();           // the previous tile's reads are done
-    if (have) put(i);
-    if (e + G < e1) fetch(e + G);
-    __syncthreads();
-    if (!have) continue;
-    const int kb = ql[e];
-    bool act = true;  // wave-uniform
-    if constexpr (HALF) act = hvalid && hrow[kb] != 0;
-    if (!act) {
-      if constexpr (EMIT) smask[size_t(e) * 256] = 0;
-      continue;
-    }
-    f32x4 acc[4];
-    for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int kat = c16 * kRs + ((8 * g) ^ Tile<u16, D>::sw(c16));
-    for (int s = 0; s < D / 32; ++s) {
-      Split8 ka[4];
-      for (int f = 0; f < 4; ++f) {
-        const int at = kat + 16 * f * kRs + 32 * s;
-        ka[f].h = *reinterpret_cast<const bf16x8*>(sm.K[0] + at);
-        ka[f].m = *reinterpret_cast<const bf16x8*>(sm.K[1] + at);
-        ka[f].l = *reinterpret_cast<const bf16x8*>(sm.K[2] + at);
-      }
-      mfma_split<4>(acc, ka, qf.v[s]);
-    }
-    const bool low = sm.low[0] == i + 1;  // group-uniform
-    if (any_nonfinite(acc) || low || qlow) {  // wave-uniform: fp32 products of the same tile
-      RowFrag<float, D> q32;
-      q32.load(qrow, qok, lane, hd);
-      rows_x_frag_global<D>(acc, Kb + size_t(kb) * kBlock * p.lk.sn, NK - kb * kBlock, size_t(p.lk.sn), hd, q32, lane);
-    }
-    auto weights = [&](auto partial) {  // as in forward_kernel
-      uint32_t nm = 0;
-      for (int f = 3; f >= 0; --f)
-        for (int r = 3; r >= 0; --r) {
-          float v = clip(acc[f][r]);
-          if constexpr (decltype(partial)::value)
-            v = sm.kid[16 * f + 4 * g + r] <= qpos ? v : -0.0f;
-          acc[f][r] = v;
-          if constexpr (EMIT) nm = __builtin_amdgcn_alignbit(nm, __float_as_uint(v), 31);
+  // The group's tiles, with scores from fp32 or from split products.  (Each
+  // walk issues its first tile's loads itself: loads shared by both cost the
+  // split one 14 registers.)
+  auto walk = [&](auto f32_tag) {
+    constexpr bool F32 = decltype(f32_tag)::value;
+    if (first < e1) fetch(first);
+    if (t == 0) sm.low[0] = 0;
+    std::conditional_t<F32, RowFrag<float, D>, SplitRow<D>> qf;
+    qf.load(qrow, qok, lane, hd);
+    bool qlow = false;  // wave-uniform
+    if constexpr (!F32) qlow = __any(split_low(qf.low));
+    // the staged quads, split, to the planes (a quad's four floats are half
+    // of a plane's 16-byte chunk); with fp32 scores K's as they are
+    auto put = [&](int step) {
+      uint32_t low = ~0u;
+      for (int i = 0; i < St::kPer; ++i) {
+        const int qi = t + i * kThreads;
+        const int job = qi / St::kQuads, qd = qi % St::kQuads;
+        const int rq = qd / St::kCpr, cc = qd % St::kCpr;
+        if (F32 && job == 0) {  // wave-uniform
+          float* dst = sm.K32 + 4 * rq * Tile<float, D>::kRs + 4 * cc;
+          for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(dst + j * Tile<float, D>::kRs) = st.r[i][j];
+          continue;
         }
-      if constexpr (EMIT) smask[size_t(e) * 256] = uint16_t(~nm);
-      for (int f = 0; f < 4; ++f)
-        for (int r = 0; r < 4; ++r) {
-          acc[f][r] = pow_clipped<PC>(acc[f][r], a);
-          rowsum += acc[f][r];
-        }
-    };
-    if (kb * kBlock + kBlock <= NK && kbnd[kb].y <= qmin) weights(std::false_type{});
-    else weights(std::true_type{});
-    if (low) {
-      for (int f = 0; f < 4; ++f)
-        for (int r = 0; r < 4; ++r) {
-          const int key = kb * kBlock + 16 * f + 4 * g + r;
-          for (int db = 0; db < D / 16; ++db) {
-            const int col = 16 * db + c16;
-            const float v = key < NK && col < hd ? Vb[size_t(key) * p.lv.sn + col] : 0.0f;
-            o[db] = mfma(v, acc[f][r], o[db]);
+        for (int j = 0; j < 4; ++j) low = split_min(low, __builtin_bit_cast(f32x4, st.r[i][j]));
+        u16* dst = (job == 0 ? sm.K[0] : sm.V[0]) + 4 * rq * kRs + ((4 * cc) ^ Tile<u16, D>::sw(4 * rq));
+        for (int j = 0; j < 4; j += 2) {
+          const Split8 x = split8(__builtin_bit_cast(f32x4, st.r[i][j]), __builtin_bit_cast(f32x4, st.r[i][j + 1]));
+          const bf16x8* pl[3] = {&x.h, &x.m, &x.l};
+          for (int y = 0; y < 3; ++y) {
+            const uint4 v = __builtin_bit_cast(uint4, *pl[y]);
+            u16* d = dst + y * (kBlock * kRs) + j * kRs;
+            *reinterpret_cast<uint2*>(d) = uint2{v.x, v.y};
+            *reinterpret_cast<uint2*>(d + kRs) = uint2{v.z, v.w};
           }
         }
-      continue;
-    }
-    for (int cc = 0; cc < 2; ++cc) {
-      const Split8 pb = split8(acc[2 * cc], acc[2 * cc + 1]);
-      const int l16 = lane & 15;
-      const int vat = (32 * cc + 4 * g + (l16 >> 2)) * kRs + ((4 * (l16 & 3)) ^ Tile<u16, D>::sw(4 * g));
-      Split8 va[D / 16];
-      auto tr = [&](int y, int db) {
-        const bf16x4 lo = read_tr16(sm.V[y] + vat + 16 * db);
-        const bf16x4 hi = read_tr16(sm.V[y] + vat + 16 * kRs + 16 * db);
-        return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      };
-      for (int db = 0; db < D / 16; ++db) {
-        va[db].h = tr(0, db);
-        va[db].m = tr(1, db);
-        va[db].l = tr(2, db);
       }
-      mfma_split<D / 16>(o, va, pb);
+      if (split_low(low)) sm.low[0] = step + 1;
+      ps.store(sm.kid, t);
+    };
+    for (int i = 0; i < steps; ++i) {
+      const int e = first + G * i;
+      const bool have = e < e1;  // group-uniform
+      __syncthreads();           // the previous tile's reads are done
+      if (have) put(i);
+      if (e + G < e1) fetch(e + G);
+      __syncthreads();
+      if (!have) continue;
+      const int kb = ql[e];
+      bool act = true;  // wave-uniform
+      if constexpr (HALF) act = hvalid && hrow[kb] != 0;
+      if (!act) {
+        if constexpr (EMIT) smask[size_t(e) * 256] = 0;
+        continue;
+      }
+      const bool low = sm.low[0] == i + 1;  // group-uniform
+      f32x4 acc[4];
+      if constexpr (F32) {
+        rows_x_frag<D>(acc, sm.K32, qf, lane);
+      } else {
+        for (int f = 0; f < 4; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int kat = c16 * kRs + ((8 * g) ^ Tile<u16, D>::sw(c16));
+        for (int s = 0; s < D / 32; ++s) {
+          Split8 ka[4];
+          for (int f = 0; f < 4; ++f) {
+            const int at = kat + 16 * f * kRs + 32 * s;
+            ka[f].h = *reinterpret_cast<const bf16x8*>(sm.K[0] + at);
+            ka[f].m = *reinterpret_cast<const bf16x8*>(sm.K[1] + at);
+            ka[f].l = *reinterpret_cast<const bf16x8*>(sm.K[2] + at);
+          }
+          mfma_split<4>(acc, ka, qf.v[s]);
+        }
+        if (any_nonfinite(acc) || low || qlow) {  // wave-uniform: fp32 products of the same tile
+          RowFrag<float, D> q32;
+          q32.load(qrow, qok, lane, hd);
+          rows_x_frag_global<D>(acc, Kb + size_t(kb) * kBlock * p.lk.sn, NK - kb * kBlock, size_t(p.lk.sn), hd, q32, lane);
+        }
+      }
+      auto weights = [&](auto partial) {  // as in forward_kernel
+        uint32_t nm = 0;
+        for (int f = 3; f >= 0; --f)
+          for (int r = 3; r >= 0; --r) {
+            float v = clip(acc[f][r]);
+            if constexpr (decltype(partial)::value)
+              v = sm.kid[16 * f + 4 * g + r] <= qpos ? v : -0.0f;
+            acc[f][r] = v;
+            if constexpr (EMIT) nm = __builtin_amdgcn_alignbit(nm, __float_as_uint(v), 31);
+          }
+        if constexpr (EMIT) smask[size_t(e) * 256] = uint16_t(~nm);
+        for (int f = 0; f < 4; ++f)
+          for (int r = 0; r < 4; ++r) {
+            acc[f][r] = pow_clipped<PC>(acc[f][r], a);
+            rowsum += acc[f][r];
+          }
+      };
+      if (kb * kBlock + kBlock <= NK && kbnd[kb].y <= qmin) weights(std::false_type{});
+      else weights(std::true_type{});
+      if (low) {
+        for (int f = 0; f < 4; ++f)
+          for (int r = 0; r < 4; ++r) {
+            const int key = kb * kBlock + 16 * f + 4 * g + r;
+            for (int db = 0; db < D / 16; ++db) {
+              const int col = 16 * db + c16;
+              const float v = key < NK && col < hd ? Vb[size_t(key) * p.lv.sn + col] : 0.0f;
+              o[db] = mfma(v, acc[f][r], o[db]);
+            }
+          }
+        continue;
+      }
+      for (int cc = 0; cc < 2; ++cc) {
+        const Split8 pb = split8(acc[2 * cc], acc[2 * cc + 1]);
+        const int l16 = lane & 15;
+        const int vat = (32 * cc + 4 * g + (l16 >> 2)) * kRs + ((4 * (l16 & 3)) ^ Tile<u16, D>::sw(4 * g));
+        Split8 va[D / 16];
+        auto tr = [&](int y, int db) {
+          const bf16x4 lo = read_tr16(sm.V[y] + vat + 16 * db);
+          const bf16x4 hi = read_tr16(sm.V[y] + vat + 16 * kRs + 16 * db);
+          return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        };
+        for (int db = 0; db < D / 16; ++db) {
+          va[db].h = tr(0, db);
+          va[db].m = tr(1, db);
+          va[db].l = tr(2, db);
+        }
+        mfma_split<D / 16>(o, va, pb);
+      }
     }
-  }
+  };
+  if (!fp32) walk(std::false_type{});
+  else walk(std::true_type{});
 
   if constexpr (G == 2) {  // the second group's sums to the first
     __syncthreads();
@@ -418,10 +457,11 @@ hipError_t launch_f32_g(const ForwardParams& p, hipStream_t s) {
   hipLaunchKernelGGL(kern, dim3(p.d.nQB * p.d.BH), dim3(G * kThreads), bytes, s, p);
   return hipGetLastError();
 }
-// The split forward applies where its output is smooth in the scores, which
-// it rounds differently (more closely) than the score pass that tau came
-// from: with k = 1 tau can lie within a rounding of the top score, and above
-// alpha = 2 the weights have unbounded slope at the support's edge.
+// The split forward rounds scores differently (more closely) than the score
+// pass that tau came from, so it applies where the output is smooth in them:
+// with k = 1 tau always lies within a rounding of the top score, and above
+// alpha = 2 the weights have unbounded slope at the support's edge.  Single
+// rows whose tau ends there (kSplitLeastU) are told apart in the kernel.
 inline bool split_ok(const ForwardParams& p) { return p.d.k >= 2 && p.d.alpha <= 2.0f; }
 
 // Two groups per block while the query blocks do not exceed the compute

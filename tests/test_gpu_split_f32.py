@@ -1,9 +1,10 @@
-"""fp32 at d <= 64: the forward's score and P V products are split bf16 products.
+"""fp32 at d <= 64: the forward's P V products are split bf16 products.
 Against the oracle at the GPU's tau (1e-5, the fp32 tolerance of the other
 parity tests), with operands whose split matters: wide magnitudes, values
-past bf16's largest; and values below 2^-109, infinities and NaN (the tiles
-that hold those run again with fp32 products).  One and two wave groups per block, few and many
-blocks, ragged lengths, a head dimension that is not a whole split step."""
+past bf16's largest; and values below 2^-109 (the tiles that hold those take
+fp32 products), infinities and NaN.  One and three wave groups per block, few
+and many blocks, ragged lengths, a head dimension that is not a whole split
+step."""
 import numpy as np
 import pytest
 import torch
@@ -16,10 +17,12 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     ("one_row", 1, 1, 1, 65, 64, 64),
-    ("two_groups_odd", 1, 2, 70, 64 * 5 + 3, 64, 64),
+    ("three_groups", 1, 2, 70, 64 * 5 + 3, 64, 64),
+    ("three_groups_odd", 1, 2, 70, 64 * 7 + 3, 64, 64),
     ("d40", 1, 2, 129, 130, 40, 64),
     ("d36_m32", 1, 2, 129, 200, 36, 32),
-    ("one_group", 3, 16, 400, 400, 64, 64),
+    ("three_groups_many", 3, 16, 400, 400, 64, 64),
+    ("one_group", 3, 16, 700, 700, 64, 64),
 ]
 
 
@@ -74,3 +77,58 @@ def test_split_error_no_larger_than_fp32_products(dev):
     e = np.linalg.norm(np32(out) - ref) / np.linalg.norm(ref)
     print(f"[split] {e:.2e}", flush=True)
     assert e < 1.5e-6
+
+
+@pytest.mark.parametrize("heads", [2, 129])
+@pytest.mark.parametrize("alpha", [1.25, 1.5, 1.7, 2.0, 2.5, 3.0])
+@pytest.mark.parametrize("k,bm", [(1, 64), (2, 64), (8, 64), (8, 32), (128, 64)])
+def test_rows_whose_best_keys_tie(dev, k, bm, alpha, heads):
+    """Keys repeated more than k times, so that a row's k best scores are equal
+    (below the clamp, inexact in fp32) and tau can end within a rounding of
+    them: the forward has to see the very scores that tau came from.  Against
+    the same call with four zero columns appended (above d = 64 nothing is
+    split, and zeros change no sum): rows without weight are the same ones,
+    support masks bit-equal.  One and two wave groups per block (heads 129
+    and 2).  The tile backward sums p over fp32 scores: each row's sum is
+    norm / (norm + 1e-8)."""
+    N, d, scale = 64 * 3 + 6, 64, 0.125
+    print(f"[split] ties k={k} bm={bm} alpha={alpha} heads={heads}", flush=True)
+    g = torch.Generator().manual_seed(int(100 * alpha) + k)
+    Q, V = (torch.randn(1, heads, N, d, generator=g) for _ in range(2))
+    # one key vector in a third of the heads, two or three in the others
+    which = torch.randint(0, 3, (1, heads, N), generator=g) % (torch.arange(heads)[None, :, None] % 3 + 1)
+    K = torch.gather(torch.randn(1, heads, 3, d, generator=g), 2, which[..., None].expand(-1, -1, -1, d))
+    qidx = torch.full((heads, N), N - 1, dtype=torch.int32, device=dev)
+    kidx = causal_idx(heads, N).to(dev)
+    q, kk, v = (t.to(dev) for t in (Q, K, V))
+    got = []
+    for pad in (0, 4):
+        p = [torch.nn.functional.pad(t, (0, pad)) for t in (q, kk, v)]
+        got.append(sa.ops.splash_forward(*p, qidx, kidx, alpha, k, scale, block_m=bm))
+    (out, st), (want, ref) = got
+    assert torch.equal(st.taus, ref.taus)
+    if bm == 64:  # the lists that index the masks are the state's
+        for h in range(heads):
+            n = int(st.q_ptr[h, -1])
+            masks = [x.sup_mask.view(torch.uint8).reshape(heads, -1, 512)[h, :n] for x in (st, ref)]
+            assert torch.equal(*masks)
+    assert bool((ref.norms < 1e-3).any())  # the draw has such rows
+    assert torch.equal(st.norms == 0, ref.norms == 0)
+    # Rows of split scores have u > 1/16, and u >= k^-1/2 at alpha = 1.5
+    # (k = 128: 0.09): u's rounding moves a weight by at most a / u = 23 times
+    # that, and (alpha - 1) times a sum of 64 products rounds by 1e-6 at most
+    # in these draws.
+    tol = 2.4e-5
+    torch.testing.assert_close(st.norms, ref.norms, rtol=tol, atol=0)
+    torch.testing.assert_close(out, want[..., :d], rtol=0, atol=tol * float(v.abs().max()))
+    # sums of p: dO with row i of a 64-row block marking column i
+    eye = torch.eye(d, device=dev).repeat(4, 1)[:N].expand(1, heads, N, d)
+    for b in range(4):
+        rows = slice(64 * b, min(64 * b + 64, N))
+        dO = torch.zeros_like(eye)
+        dO[:, :, rows] = eye[:, :, rows]
+        st.sup_mask = None  # the tile passes
+        _, _, dV = sa.ops.splash_backward(q, kk, v, qidx, kidx, out, dO, st, alpha, k, scale)
+        sums = dV.sum(2)[0, :, :rows.stop - rows.start]
+        norms = st.norms.view(heads, N)[:, rows]
+        torch.testing.assert_close(sums, norms / (norms + 1e-8), rtol=0, atol=tol)
