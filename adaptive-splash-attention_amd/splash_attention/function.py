@@ -31,9 +31,10 @@ class SplashAttentionFunction(torch.autograd.Function):
                                                    and bwd_passes == "support"),
                                      tau_mode=tau_mode, block_m=block_m)
         ctx.params = (alpha, k_keep, sm_scale, grad_mode)
-        # the output only where the backward reads it (the reference gradient)
-        ctx.save_for_backward(Q, K, V, Q_idx, K_idx, out if grad_mode == "reference" else None,
-                              *st.tensors())
+        # the output too where the backward does not read it (the entmax
+        # gradient): an in-place change of it before backward is then refused
+        # in both gradient modes, as through the custom operator
+        ctx.save_for_backward(Q, K, V, Q_idx, K_idx, out, *st.tensors())
         return out
 
     @staticmethod

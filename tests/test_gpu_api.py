@@ -225,3 +225,16 @@ def test_non_contiguous_inputs(dev):
     a = sa.forward(qt, kt, vt, idx, idx, 0.125, 1.5)
     b = sa.forward(Q.to(dev), K.to(dev), V.to(dev), idx, idx, 0.125, 1.5)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("grad_mode", ["entmax", "reference"])
+def test_output_changed_in_place_before_backward_is_refused(dev, grad_mode):
+    """The output is part of what the backward is promised, in both gradient
+    modes (eagerly as through the custom operator)."""
+    print(f"[api] in-place {grad_mode}", flush=True)
+    Q, K, V, _ = make_inputs(1, 1, 70, 70, 64, seed=5)
+    q, k, v = (t.to(dev).requires_grad_(True) for t in (Q, K, V))
+    out = sa.splash_attention(q, k, v, grad_mode=grad_mode)
+    out.mul_(2.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
