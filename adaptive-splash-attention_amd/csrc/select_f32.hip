@@ -28,18 +28,25 @@ SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_ld
   const bool wide = raw && (few || d.k > 64 || (d.k > 42 && ring && d.D == 128)) &&
                     !(dtype == kElemF32 && d.D == 128);
   const struct { int waves; bool ring; } tries[] = {{wide ? 8 : 4, ring}, {4, ring}, {4, false}};
+  // k + 32 keys per row hold the candidates of random rows with room to
+  // spare up to k = 42, and 1.75 k above (the floor's slack grows with k).
+  // Where LDS is short (the visible list takes 4 bytes per key block) the
+  // first variant that holds k + k / 8 + 16 is taken (random rows list about
+  // 1.15 k), else the one that holds most.  Less still works, by overflow
+  // rounds that drop cap - k keys each, down to k + 4.
+  SelectPlan plan{4, false, -1, 0};
   for (const auto& t : tries) {
     auto bytes = [&](int cap) { return size_t(sel_layout(d.k, cap, d.nKB, t.waves, t.ring ? d.D : 0).total); };
-    // k + 32 keys per row hold the candidates of random rows with room to
-    // spare up to k = 42, and 1.75 k above (the floor's slack grows with
-    // k); less still works (overflow rounds), as long as it exceeds k.
     int cap = d.k + (d.k * 3 / 4 > 32 ? d.k * 3 / 4 : 32);
-    while (cap > d.k && bytes(cap) > max_lds) cap -= 4;
-    if (cap <= d.k) cap = d.k + 4;  // the least taken
-    if (bytes(cap) <= max_lds) return SelectPlan{t.waves, t.ring, cap, 0};
-    if (t.waves == 4 && !t.ring) return SelectPlan{4, false, -1, bytes(cap)};
+    while (cap > d.k + 4 && bytes(cap) > max_lds) cap = cap - 4 > d.k + 4 ? cap - 4 : d.k + 4;
+    if (bytes(cap) > max_lds) {
+      if (plan.cap < 0) plan.needs = bytes(cap);
+      continue;
+    }
+    if (cap > plan.cap) plan = SelectPlan{t.waves, t.ring, cap, 0};
+    if (cap >= d.k + d.k / 8 + 16) break;
   }
-  return SelectPlan{4, false, -1, 0};
+  return plan;
 }
 
 }  // namespace asa
