@@ -254,7 +254,10 @@ __global__ __launch_bounds__(kThreads, 4) void dq_sparse_kernel(BackwardParams p
     if (qrow < NQ) {
       const size_t rw = size_t(bh) * NQ + qrow;
       nrm = p.norms[rw];
-      ta = p.taus[rw];
+      // A row without weight can list pairs (u = 0 exactly, where its best
+      // scores tie at tau), and u as recomputed here can be above 0: with
+      // tau = inf nothing of the row passes, here and in the dK/dV pass.
+      ta = nrm == 0.0f ? __builtin_inff() : p.taus[rw];
       if constexpr (REF) {
         c = p.delta[rows + rw];
         sh = p.delta[rw];

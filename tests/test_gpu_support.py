@@ -75,3 +75,27 @@ def test_support_masks_match_dense_scores(dev, dtype):
 def test_support_masks_nq_ne_nk_alpha2(dev):
     print("[support] 2x1x130x257 d128 alpha 2", flush=True)
     _support_check(dev, 2, 1, 130, 257, 128, 2.0, 8, 128 ** -0.5, torch.bfloat16, seed=32)
+
+
+@pytest.mark.parametrize("mode", ["entmax", "reference"])
+@pytest.mark.parametrize("alpha,k", [(1.5, 8), (2.0, 2), (2.0, 8), (3.0, 8), (1.5, 1)])
+@pytest.mark.parametrize("d,dtype", [(64, torch.float32), (128, torch.float32), (64, torch.bfloat16),
+                                     (80, torch.float16), (128, torch.bfloat16)])
+def test_rows_without_weight_give_no_gradient(dev, d, dtype, alpha, k, mode):
+    """Rows whose best scores tie at tau (one key vector, repeated) can have no
+    weight at all: their output and dQ are 0, and they add nothing to dK and
+    dV.  dO is nonzero in such rows only, so every gradient is exactly 0."""
+    B, H, N = 1, 3, 64 * 3 + 6
+    print(f"[support] no weight d{d} {dtype} alpha {alpha} k {k} {mode}", flush=True)
+    Q, K, V, dO = make_inputs(B, H, N, N, d, seed=d + k)
+    K = K[:, :, :1].expand(-1, -1, N, -1).contiguous()
+    q, kk, v, g = (t.to(dtype).to(dev) for t in (Q, K, V, dO))
+    qi = torch.full((B * H, N), N - 1, dtype=torch.int32, device=dev)
+    ki = causal_idx(B * H, N).to(dev)
+    out, st = sa.ops.splash_forward(q, kk, v, qi, ki, alpha, k, d ** -0.5)
+    none = (st.norms == 0).view(B, H, N, 1)
+    assert bool(none.any())
+    assert not bool((out * none).any())
+    grads = sa.ops.splash_backward(q, kk, v, qi, ki, out, g * none, st, alpha, k, d ** -0.5, mode)
+    for name, t in zip(("dQ", "dK", "dV"), grads):
+        assert not bool(t.any()), f"{name}: largest {float(t.abs().max()):.2e}"
