@@ -267,3 +267,47 @@ def test_score_pass_by_block_count(dev, d, dtype, k, NK, heads):
             x, want = getattr(st, name).cpu().numpy(), getattr(sel, name)
             for h in range(heads):
                 np.testing.assert_array_equal(x[h], want[h % 2])
+
+
+@pytest.mark.parametrize("d,dtype,k,heads", [
+    (64, torch.bfloat16, 32, 3), (64, torch.bfloat16, 32, 257), (64, torch.float16, 128, 3),
+    (128, torch.bfloat16, 64, 3), (128, torch.float16, 32, 257), (80, torch.bfloat16, 64, 257),
+    (64, torch.float32, 64, 3), (64, torch.float32, 8, 257)])
+def test_operand_overflow_rounds(dev, d, dtype, k, heads):
+    """Overflow rounds with the scores formed from Q and K (rings or register
+    loads, four or eight waves per block, 3 or 257 blocks): head 0 has
+    _rising_scores' pattern, head 1 half of its keys tied at the score clamp
+    and the others just below, head 2 both.  Against the oracle, on scores
+    that are exact in fp32."""
+    import splash_attention as sa
+
+    NQ, NK, scale = 64, 2048 + 37, 0.125
+    print(f"[select] operand overflow d={d} {dtype} k={k} heads={heads}", flush=True)
+    j = np.arange(NK)
+    high = j % 64 < (k - 1) // (2 if k <= 64 else 4)
+    rng = np.random.default_rng(d + k)
+    raw = [np.where(high, 16 + j / 128, -8 - j / 128),       # 2 .. 4.1 after scaling
+           np.where(rng.random(NK) < 0.5, 96, 64 + j / 128),  # 10 (clamped) or 8 ..
+           np.where(high, 48 + j / 64, np.where(rng.random(NK) < 0.5, 40, -8))]
+    # raw = its floor + a multiple of 1/128, each exact in 16 bits
+    K = np.zeros((1, 3, NK, d), np.float32)
+    for h in range(3):
+        K[0, h, :, 0], K[0, h, :, d - 1] = np.floor(raw[h]), raw[h] - np.floor(raw[h])
+    Q = np.zeros((1, 3, NQ, d), np.float32)
+    Q[..., 0] = Q[..., d - 1] = 1.0
+    kidx = causal_idx(heads, NK)
+    qidx = (NK - 1 - 3 * torch.arange(NQ, dtype=torch.int32)).expand(heads, NQ).contiguous()
+    rep = torch.arange(heads) % 3
+    q, kk = (torch.from_numpy(x)[:, rep].contiguous().to(dtype).to(dev) for x in (Q, K))
+    got = [sa.ops.splash_forward(q, kk, kk, qidx.to(dev), kidx.to(dev), 1.5, k, scale,
+                                 with_topk=t, with_support=False)[1] for t in (True, False)]
+    rounds = [st.overflow_rounds() for st in got]
+    print(f"[select] operand overflow: {rounds} rounds", flush=True)
+    S, vis = orc.scores(Q[0], K[0], qidx[:3].numpy(), kidx[:3].numpy(), scale)
+    sel = orc.select(S, vis, k, 1.5)
+    for st, n in zip(got, rounds):
+        assert n >= 1 and not st.status_word() & sa._lib.STATUS_SELECT_ROUNDS
+        for name in ("mask", "taus") + (("topk_idx", "topk_val") if st.topk_idx is not None else ()):
+            x, want = getattr(st, name).cpu().numpy(), getattr(sel, name)
+            for h in range(heads):
+                np.testing.assert_array_equal(x[h], want[h % 3])
