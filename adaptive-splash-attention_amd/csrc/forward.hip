@@ -201,14 +201,16 @@ constexpr float kSplitLeastU = 0x1p-4f;
 // bf16 planes once, as they are staged (55 KB of LDS for one tile pair: two
 // blocks per compute unit; the next pair loads into registers meanwhile),
 // the weights in registers; the scores and P V then take 96 matrix products
-// per tile and wave at 16 cycles instead of 128 at 32.  The splitting (about
-// 330 VALU instructions per tile and wave) and the planes' LDS reads (48 KB)
-// take about as long as the products.  G = 2: two groups of four waves take
+// per tile and wave at 16 cycles instead of 128 at 32.  About 770 VALU
+// instructions per tile and wave (by counters; mostly the splitting) and the
+// planes' LDS reads (48 KB) take longer than the products: the matrix unit is
+// 13% busy at 1x4x4096.  G = 2: two groups of four waves take
 // every other tile of the list, and the second one's sums are added to the
 // first one's at the end, where the query blocks alone leave compute units
 // with one wave per SIMD.  Measured against forward_kernel: 4x16x4096x64
-// 1249 -> 980 us, 2x8x2048x64 125 -> 102 us, 1x4x4096x64 219 -> 150 us; the
-// output's 2-norm error against float64 falls from 1.2e-6 to 0.8e-6.
+// 1245 -> 1020 us, 2x8x2048x64 125 -> 106 us, 1x4x4096x64 217 -> 153 us; the
+// output's 2-norm error against float64 at equal tau (1x4x4096, alpha 1.5,
+// k = 8) falls from 6.9e-7 to 4.4e-7.
 template <int D> struct alignas(16) SplitFwdSmem {
   union {
     u16 K[3][kBlock * Tile<u16, D>::kRs];

@@ -19,11 +19,12 @@ SelectPlan select_plan(const Dims& d, int dtype, bool from_scores, size_t max_ld
   // with eight).  1x8x32768, d = 128, k = 128: 4.9 -> 3.7 ms.  fp32 at
   // d = 128 holds 128 registers of Q and would spill at two waves per SIMD.
   // And where the grid gives each compute unit one block at most, whose
-  // waves then are all that the unit runs: calls of four against eight
-  // waves, 16x16 heads of 1x4096, d = 64, k = 32, bf16 104.1 -> 97.7 us;
-  // fp32, d = 64, k = 8: forward at 1x4x4096 402 -> 375 us, backward (with
-  // its forward) at 1x6x1500 281 -> 271 us.  With more blocks two 4-wave
-  // ones share a unit.
+  // waves then are all that the unit runs: this kernel with four against
+  // eight waves, 1x4x4096, k = 32: bf16 d = 64 67 -> 45 us, d = 128 79 -> 56,
+  // d = 80 80 -> 53, fp16 d = 128 79 -> 56, fp32 d = 64 180 -> 161; 1x2x1500
+  // bf16 d = 128 46 -> 33; 16x16 heads of 1x4096, bf16 d = 64 54 -> 48,
+  // d = 128 90 -> 92 (each block streams its own K there).  With more blocks
+  // two 4-wave ones share a unit.
   const bool few = size_t(d.nQB) * size_t(d.BH) <= size_t(cus);
   const bool wide = raw && (few || d.k > 64 || (d.k > 42 && ring && d.D == 128)) &&
                     !(dtype == kElemF32 && d.D == 128);

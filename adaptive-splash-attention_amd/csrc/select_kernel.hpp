@@ -229,19 +229,20 @@ enum KLayout : int { kKDense = 0, kKRows = 1, kKGeneral = 2 };
 // (c, g) holds key 16 w + c at the head-dimension slots that rows_x_frag
 // gives lane group g.  product() forms, for each of the four 16-row groups
 // cb of the query block, the scores of the quarter's keys against rows
-// 16 cb + c with the same operands in the same accumulation order as the
-// attention passes' rows_x_frag, so every score is bit-identical to theirs.
+// 16 cb + c with the same operands in the same accumulation order as
+// rows_x_frag, so every score is bit-identical to those of the passes that use
+// it: the forward (but for fp32 at d <= 64, whose split products round
+// otherwise; kSplitLeastU) and the tile backward.
 // acc[cb][r] is the score of key 16 w + 4 g + r and row 16 cb + c.
 template <typename T, int D> struct KQuarter;
 template <typename T, int D> struct KQuarter16 {
   using V8 = typename Half<T>::v8;
   V8 a[D / 32];
   // `src`: the tile's first row plus the lane's byte offset (its key's row,
-  // 16 g bytes in).  (This register path loads 16 half rows per instruction,
-  // a third of the L2 rate of whole-row loads; a whole-row load with the
-  // operands rebuilt by two DPP row rotations per register measured the same
-  // sweep time, which the candidate appends, not the loads, set.)  KL
-  // (KLayout): with kKGeneral columns >= hd read as zero.
+  // 16 g bytes in).  This register path loads 16 half rows per instruction,
+  // a third of the L2 rate of whole-row loads; the rings (sweep_ring) read
+  // whole rows where hd = D.  KL (KLayout): with kKGeneral columns >= hd read
+  // as zero.
   template <int KL>
   __device__ __forceinline__ void load(const unsigned char* tile, uint32_t off, int hd, int g) {
     for (int s = 0; s < D / 32; ++s)
