@@ -311,8 +311,9 @@ __device__ __forceinline__ void tile_t_x_acc(f32x4 (&o)[D / 16], const float* rm
 // v_mfma_f32_16x16x32_bf16 take 96 cycles where eight
 // v_mfma_f32_16x16x4_f32 take 256.  |x| beyond bf16's largest value is
 // clamped into h, so that m and l carry the rest; an infinity or a NaN makes
-// l a NaN, and every product of it a NaN.  Tiles with a non-finite score or
-// an operand below 2^-109 (split_low) run again with fp32 products.
+// l a NaN, and every product of it a NaN.  A wave with a non-finite score
+// takes fp32 products for that tile's scores, a block with an operand below
+// 2^-109 (split_low) fp32 products from there on.
 // ---------------------------------------------------------------------------
 struct Split8 {
   bf16x8 h, m, l;

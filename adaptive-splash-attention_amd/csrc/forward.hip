@@ -184,7 +184,7 @@ __global__ __launch_bounds__(kThreads) void forward_kernel(ForwardParams p) {
 }
 
 // Blocks with a row whose best key has u = (alpha - 1) s - tau of at most this
-// take fp32 products for their scores, the rounding that tau came from.  Where
+// take fp32 products, the rounding that tau came from.  Where
 // a row's k best scores are equal (repeated keys) the threshold recurrence
 // starts within a rounding of them and can end there, and the score's rounding
 // then decides whether the row has any weight (alpha = 2: no output, or the
@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kThreads) void forward_kernel(ForwardParams p) {
 // Below the line are rows whose recurrence did not converge in its five rounds
 // and nearly uniform ones: more than 16 equal weights at alpha = 2, 256 at
 // 1.5.  Such a block costs what forward_kernel's does (2x8x2048x64, alpha 2,
-// k = 128, 0.1 N(0, 1): 123 us, forward_kernel 128, split scores 107).
+// k = 128, 0.1 N(0, 1): 132 us, forward_kernel 128, split products 107).
 constexpr float kSplitLeastU = 0x1p-4f;
 
 // fp32 at d <= 64 (split_ok): the one-block kernel on the bf16 matrix unit
@@ -208,17 +208,23 @@ constexpr float kSplitLeastU = 0x1p-4f;
 // every other tile of the list, and the second one's sums are added to the
 // first one's at the end, where the query blocks alone leave compute units
 // with one wave per SIMD.  Measured against forward_kernel: 4x16x4096x64
-// 1245 -> 1020 us, 2x8x2048x64 125 -> 106 us, 1x4x4096x64 217 -> 153 us; the
+// 1245 -> 1036 us, 2x8x2048x64 125 -> 107 us, 1x4x4096x64 217 -> 154 us; the
 // output's 2-norm error against float64 at equal tau (1x4x4096, alpha 1.5,
-// k = 8) falls from 6.9e-7 to 4.4e-7.
+// k = 8) falls from 6.9e-7 to 4.4e-7.  From the first tile with a value below
+// 2^-109 on, a block goes on with fp32 products of the tiles as they are: such
+// values in every tile of 4x16x2048x64 take 359 to 378 us (forward_kernel 331
+// to 346, split products 298; 950 to 1040 with such tiles done one by one).
 template <int D> struct alignas(16) SplitFwdSmem {
   union {
     u16 K[3][kBlock * Tile<u16, D>::kRs];
-    float K32[kBlock * Tile<float, D>::kRs];  // blocks with fp32 scores
+    float K32[kBlock * Tile<float, D>::kRs];  // with fp32 products
   };
-  u16 V[3][kBlock * Tile<u16, D>::kRs];
+  union {
+    u16 V[3][kBlock * Tile<u16, D>::kRs];
+    float V32[kBlock * Tile<float, D>::kRs];
+  };
   int kid[kBlock];
-  int low[4];  // low[0]: 1 + the last step whose tiles hold a value below 2^-109
+  int low[4];  // low[0]: 1 + the step whose tiles (or, at 0, Q rows) hold a value below 2^-109
 };
 
 template <int D, int PC, bool EMIT, bool HALF, int G>
@@ -248,7 +254,7 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
   const float a = 1.0f / am1;
   const SignedClip clip(am1, p.d.scale, qok ? p.taus[row] : 0.0f, qok);  // invalid rows: p = 0
   // as in forward_kernel: key blocks up to qmin are visible to every row;
-  // and whether the block takes fp32 scores (kSplitLeastU)
+  // and whether the block takes fp32 products (kSplitLeastU)
   int qmin;
   bool fp32;  // block-uniform
   {
@@ -284,35 +290,33 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
     ps.load(kidx, kbase, NK, INT32_MAX, t);
   };
   const int first = e0 + grp, steps = (e1 - e0 + G - 1) / G;  // block-uniform
-  // The group's tiles, with scores from fp32 or from split products.  (Each
-  // walk issues its first tile's loads itself: loads shared by both cost the
-  // split one 14 registers.)
-  auto walk = [&](auto f32_tag) {
+  if (t == 0) sm.low[0] = 0;
+  // The group's tiles from step i on, with fp32 or with split products; the
+  // split walk returns before the first step where a K or V tile (or, before
+  // step 0, a Q row) holds a value below the split's range.  (Each walk issues its first
+  // tile's loads itself: loads shared by both cost the split one 14
+  // registers.)
+  auto walk = [&](auto f32_tag, int i) {
     constexpr bool F32 = decltype(f32_tag)::value;
-    if (first < e1) fetch(first);
-    if (t == 0) sm.low[0] = 0;
+    if (first + G * i < e1) fetch(first + G * i);
     std::conditional_t<F32, RowFrag<float, D>, SplitRow<D>> qf;
     qf.load(qrow, qok, lane, hd);
-    bool qlow = false;  // wave-uniform
-    if constexpr (!F32) qlow = __any(split_low(qf.low));
     // the staged quads, split, to the planes (a quad's four floats are half
-    // of a plane's 16-byte chunk); with fp32 scores K's as they are
+    // of a plane's 16-byte chunk)
     auto put = [&](int step) {
       uint32_t low = ~0u;
-      for (int i = 0; i < St::kPer; ++i) {
-        const int qi = t + i * kThreads;
+      if constexpr (!F32) low = step == 0 ? qf.low : ~0u;
+      for (int x = 0; x < St::kPer; ++x)
+        for (int j = 0; j < 4; ++j) low = split_min(low, __builtin_bit_cast(f32x4, st.r[x][j]));
+      if (split_low(low)) sm.low[0] = step + 1;
+      for (int x = 0; x < St::kPer; ++x) {
+        const int qi = t + x * kThreads;
         const int job = qi / St::kQuads, qd = qi % St::kQuads;
         const int rq = qd / St::kCpr, cc = qd % St::kCpr;
-        if (F32 && job == 0) {  // wave-uniform
-          float* dst = sm.K32 + 4 * rq * Tile<float, D>::kRs + 4 * cc;
-          for (int j = 0; j < 4; ++j) *reinterpret_cast<uint4*>(dst + j * Tile<float, D>::kRs) = st.r[i][j];
-          continue;
-        }
-        for (int j = 0; j < 4; ++j) low = split_min(low, __builtin_bit_cast(f32x4, st.r[i][j]));
         u16* dst = (job == 0 ? sm.K[0] : sm.V[0]) + 4 * rq * kRs + ((4 * cc) ^ Tile<u16, D>::sw(4 * rq));
         for (int j = 0; j < 4; j += 2) {
-          const Split8 x = split8(__builtin_bit_cast(f32x4, st.r[i][j]), __builtin_bit_cast(f32x4, st.r[i][j + 1]));
-          const bf16x8* pl[3] = {&x.h, &x.m, &x.l};
+          const Split8 sp = split8(__builtin_bit_cast(f32x4, st.r[x][j]), __builtin_bit_cast(f32x4, st.r[x][j + 1]));
+          const bf16x8* pl[3] = {&sp.h, &sp.m, &sp.l};
           for (int y = 0; y < 3; ++y) {
             const uint4 v = __builtin_bit_cast(uint4, *pl[y]);
             u16* d = dst + y * (kBlock * kRs) + j * kRs;
@@ -321,16 +325,23 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
           }
         }
       }
-      if (split_low(low)) sm.low[0] = step + 1;
-      ps.store(sm.kid, t);
     };
-    for (int i = 0; i < steps; ++i) {
+    for (; i < steps; ++i) {
       const int e = first + G * i;
       const bool have = e < e1;  // group-uniform
       __syncthreads();           // the previous tile's reads are done
-      if (have) put(i);
+      if (have) {
+        if constexpr (F32) st.store(sm.K32, sm.V32, t);
+        else put(i);
+        ps.store(sm.kid, t);
+      }
       if (e + G < e1) fetch(e + G);
       __syncthreads();
+      if constexpr (!F32) {
+        bool low = false;  // block-uniform
+        for (int y = 0; y < G; ++y) low |= reinterpret_cast<SplitFwdSmem<D>*>(smem_split)[y].low[0] == i + 1;
+        if (low) break;
+      }
       if (!have) continue;
       const int kb = ql[e];
       bool act = true;  // wave-uniform
@@ -339,7 +350,6 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
         if constexpr (EMIT) smask[size_t(e) * 256] = 0;
         continue;
       }
-      const bool low = sm.low[0] == i + 1;  // group-uniform
       f32x4 acc[4];
       if constexpr (F32) {
         rows_x_frag<D>(acc, sm.K32, qf, lane);
@@ -356,7 +366,7 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
           }
           mfma_split<4>(acc, ka, qf.v[s]);
         }
-        if (any_nonfinite(acc) || low || qlow) {  // wave-uniform: fp32 products of the same tile
+        if (any_nonfinite(acc)) {  // wave-uniform: fp32 products of the same tile
           RowFrag<float, D> q32;
           q32.load(qrow, qok, lane, hd);
           rows_x_frag_global<D>(acc, Kb + size_t(kb) * kBlock * p.lk.sn, NK - kb * kBlock, size_t(p.lk.sn), hd, q32, lane);
@@ -381,39 +391,33 @@ __global__ __launch_bounds__(G * kThreads) void forward_kernel(ForwardParams p) 
       };
       if (kb * kBlock + kBlock <= NK && kbnd[kb].y <= qmin) weights(std::false_type{});
       else weights(std::true_type{});
-      if (low) {
-        for (int f = 0; f < 4; ++f)
-          for (int r = 0; r < 4; ++r) {
-            const int key = kb * kBlock + 16 * f + 4 * g + r;
-            for (int db = 0; db < D / 16; ++db) {
-              const int col = 16 * db + c16;
-              const float v = key < NK && col < hd ? Vb[size_t(key) * p.lv.sn + col] : 0.0f;
-              o[db] = mfma(v, acc[f][r], o[db]);
-            }
+      if constexpr (F32) {
+        tile_t_x_acc<D>(o, sm.V32, acc, lane);
+      } else {
+        for (int cc = 0; cc < 2; ++cc) {
+          const Split8 pb = split8(acc[2 * cc], acc[2 * cc + 1]);
+          const int l16 = lane & 15;
+          const int vat = (32 * cc + 4 * g + (l16 >> 2)) * kRs + ((4 * (l16 & 3)) ^ Tile<u16, D>::sw(4 * g));
+          Split8 va[D / 16];
+          auto tr = [&](int y, int db) {
+            const bf16x4 lo = read_tr16(sm.V[y] + vat + 16 * db);
+            const bf16x4 hi = read_tr16(sm.V[y] + vat + 16 * kRs + 16 * db);
+            return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          };
+          for (int db = 0; db < D / 16; ++db) {
+            va[db].h = tr(0, db);
+            va[db].m = tr(1, db);
+            va[db].l = tr(2, db);
           }
-        continue;
-      }
-      for (int cc = 0; cc < 2; ++cc) {
-        const Split8 pb = split8(acc[2 * cc], acc[2 * cc + 1]);
-        const int l16 = lane & 15;
-        const int vat = (32 * cc + 4 * g + (l16 >> 2)) * kRs + ((4 * (l16 & 3)) ^ Tile<u16, D>::sw(4 * g));
-        Split8 va[D / 16];
-        auto tr = [&](int y, int db) {
-          const bf16x4 lo = read_tr16(sm.V[y] + vat + 16 * db);
-          const bf16x4 hi = read_tr16(sm.V[y] + vat + 16 * kRs + 16 * db);
-          return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        };
-        for (int db = 0; db < D / 16; ++db) {
-          va[db].h = tr(0, db);
-          va[db].m = tr(1, db);
-          va[db].l = tr(2, db);
+          mfma_split<D / 16>(o, va, pb);
         }
-        mfma_split<D / 16>(o, va, pb);
       }
     }
+    return i;
   };
-  if (!fp32) walk(std::false_type{});
-  else walk(std::true_type{});
+  int i = 0;
+  if (!fp32) i = walk(std::false_type{}, i);
+  if (i < steps) walk(std::true_type{}, i);
 
   if constexpr (G == 2) {  // the second group's sums to the first
     __syncthreads();

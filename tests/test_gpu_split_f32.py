@@ -1,8 +1,8 @@
 """fp32 at d <= 64: the forward's score and P V products are split bf16 products.
 Against the oracle at the GPU's tau (1e-5, the fp32 tolerance of the other
 parity tests), with operands whose split matters: wide magnitudes, values
-past bf16's largest; and values below 2^-109, infinities and NaN (the tiles
-that hold those run again with fp32 products).  One and two wave groups per
+past bf16's largest; and values below 2^-109, infinities and NaN (fp32
+products from there on, or for that tile).  One and two wave groups per
 block, few and many blocks, ragged lengths, a head dimension that is not a
 whole split step.  Rows whose best scores tie at tau."""
 import numpy as np
@@ -25,7 +25,7 @@ CASES = [
 
 
 @pytest.mark.parametrize("alpha", [1.5, 1.25, 1.7, 2.0])
-@pytest.mark.parametrize("kind", ["normal", "wide", "huge", "tiny", "nonfinite"])
+@pytest.mark.parametrize("kind", ["normal", "wide", "huge", "tiny", "nonfinite", "low_tile", "low_row"])
 @pytest.mark.parametrize("name,B,H,NQ,NK,d,bm", CASES, ids=[c[0] for c in CASES])
 def test_split_forward(dev, name, B, H, NQ, NK, d, bm, kind, alpha):
     print(f"[split] {name} {kind} B{B} H{H} NQ{NQ} NK{NK} d{d} block_m {bm} alpha {alpha}", flush=True)
@@ -40,6 +40,11 @@ def test_split_forward(dev, name, B, H, NQ, NK, d, bm, kind, alpha):
         Q[..., 0] *= 1e-38             # and values below the split's range
     elif kind == "tiny":
         V *= 1e-37
+    elif kind == "low_tile":  # one value below 2^-109 late in the lists: split products until there
+        K[:, ::2, NK // 2, 5] = 1e-35
+        V[:, 1::2, 2 * NK // 3, 7] = -1e-38
+    elif kind == "low_row":   # and in one row of Q
+        Q[:, :, NQ // 2, 9] = 1e-36
     elif kind == "nonfinite":
         K[:, :, NK // 2, 0] = float("inf")
         K[:, :, NK // 3, 1] = float("nan")
