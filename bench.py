@@ -57,8 +57,8 @@ COPY_BYTES = 256 << 20   # --copy-calibration copy size
 # library built from the sources whose hash is HBM_TRAFFIC_SOURCES
 # (source_hash()).  A line from a library built from other sources reports
 # traffic null and says why: counters of another build are not evidence.
-HBM_TRAFFIC_SOURCES = "98d3f9411e609781"
-HBM_TRAFFIC = {'bounds': 1109721, 'select': 141281244, 'tau': 34740395, 'tau_compact': 37523563, 'refine': 109842411, 'compact': 2761045, 'forward': 330738293, 'bwd_dq_sparse': 240754196, 'bwd_dkdv_sparse': 287731744}
+HBM_TRAFFIC_SOURCES = "29048bb7d45382c7"
+HBM_TRAFFIC = {'bounds': 1110674, 'select': 141539022, 'tau': 34740416, 'tau_compact': 37521280, 'refine': 109852944, 'compact': 2761045, 'forward': 330553433, 'bwd_dq_sparse': 240731648, 'bwd_dkdv_sparse': 287763040}
 
 
 def source_hash() -> str:
